@@ -84,8 +84,10 @@ typedef struct {
  * (unpadded planes) whenever its tile fits the LDS, else the ghost-padded
  * global gather; GHOST forces the latter.  Results agree to rounding.  AUTO
  * also takes the ghost layout for one replica of 513 to 8192 sites without
- * Ewald, whose midpoint steps then run in one cooperative launch per call
- * (snh_query "cooperative"). */
+ * Ewald.  One replica of 513 to 28,672 sites without Ewald, on either layout,
+ * runs the midpoint steps of a call and calls of several Langevin steps in
+ * one cooperative launch (snh_query "cooperative"; SNH_COOP=0 at snh_create
+ * launches every stage, SNH_COOP_MAX_SITES lowers the bound). */
 #define SNH_LAYOUT_AUTO 0
 #define SNH_LAYOUT_GHOST 1
 

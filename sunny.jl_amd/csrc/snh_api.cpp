@@ -462,13 +462,15 @@ struct SystemImpl final : snh_system {
     int* pinned_i = nullptr;   // [R]
     int planes = 3;
     int last_iters = 4;
-    // Small :dipole replicas on the ghost layout (no Ewald) step in one
-    // persistent workgroup per replica: no launch per stage, no host check
-    bool coop = false;  // cooperative midpoint launch (one replica, ghost layout)
-    double* coop_partial = nullptr;  // [2 nblocks]
-    unsigned* coop_bar = nullptr;    // count, gen, err
-    // per midpoint step.
-    bool persist = false;
+    // Small :dipole replicas on the ghost layout (no Ewald) step inside one
+    // launch per call: no launch per stage, no host check per midpoint step.
+    bool persist = false;  // every replica is one workgroup
+    bool coop = false;     // one replica (either layout) cut into parts, one workgroup each, all resident
+    ResPlan res;
+    ResArgs res_args{};
+    unsigned long long* res_ex = nullptr;  // exchanged words of a launch
+    int* res_err = nullptr;                // host memory: a wait of some launch timed out
+    T* res_sdd = nullptr;                  // where a resident midpoint leaves S'' (the adjoint's recording)
     // Tiled Langevin batches of two or more replicas (no Ewald) step as two
     // replica groups on two streams in anti-phase: one group's corrector
     // (latency-bound) runs beside the other's predictor (VALU-bound).
@@ -481,7 +483,7 @@ struct SystemImpl final : snh_system {
     int64_t mid_fallbacks = 0;  // midpoint step groups then run with per-step host checks
     hipStream_t st2 = nullptr;
     hipEvent_t pev[3] = {nullptr, nullptr, nullptr};  // start, first group's predictor, second group's predictor
-    int* fail_step = nullptr;  // [R] persistent midpoint / budgeted groups: step that did not converge
+    int* fail_step = nullptr;  // [R] resident midpoint / budgeted groups: step that did not converge
     int* max_iter = nullptr;   // [R] budgeted midpoint groups: largest iteration count
     // Sampled correlations of one :dipole replica (snh_corr.hip)
     struct Corr {
@@ -573,7 +575,57 @@ struct SystemImpl final : snh_system {
         for (void* p : owned) (void)hipFree(p);
         if (pinned) (void)hipHostFree(pinned);
         if (pinned_i) (void)hipHostFree(pinned_i);
+        if (res_err) (void)hipHostFree(res_err);
         if (st) (void)hipStreamDestroy(st);
+    }
+
+    // Plan and device tables of the resident launches; a handle without a
+    // plan takes the launch per stage.
+    void build_resident(const std::vector<int>& bstart)
+    {
+        hipDeviceProp_t prop;
+        SNH_HIP(hipGetDeviceProperties(&prop, dev));
+        std::vector<std::array<int, 3>> dims;
+        for (const auto& ri : reps) dims.push_back({ri.L1, ri.L2, ri.L3});
+        std::vector<std::array<int, 4>> slots(std::max(nb, 1));
+        for (int i = 0; i < na; i++)
+            for (int k = bstart[i]; k < bstart[i + 1]; k++) {
+                const int32_t* bd = bsrc_h[k] < 0 ? nullptr : bond_h.data() + 6 * (size_t)bsrc_h[k];
+                slots[k] = bd ? std::array<int, 4>{bd[2], bd[3], bd[4], bd[1]} : std::array<int, 4>{0, 0, 0, i};
+            }
+        // 256 bytes stay free for the kernels' static LDS
+        if (!plan_resident(na, dims, bstart, slots, sizeof(T), prop.sharedMemPerBlock - 256, res)) {
+            persist = coop = false;
+            return;
+        }
+        if (res.halo.empty()) res.halo.push_back(0);
+        if (res.nbr.empty()) res.nbr.push_back(0);
+        ResArgs& A = res_args;
+        A.wg = own(dupload(res.wg));
+        A.lane = own(dupload(res.lane));
+        A.halo = own(dupload(res.halo));
+        A.nbr = own(dupload(res.nbr));
+        const size_t words = res_words(res, sizeof(T));
+        if (words) res_ex = own(dalloc<unsigned long long>(words));
+        A.ex = res_ex;
+        A.res = res_ex ? res_ex + words - 4 * (size_t)res.nres : nullptr;
+        A.nslot = res.nslot;
+        A.nex = res.nex;
+        A.nres = res.nres;
+        A.spin = 1u << 22;
+        SNH_HIP(hipHostMalloc((void**)&res_err, sizeof(int), hipHostMallocDefault));
+        *res_err = 0;
+        A.err = res_err;
+        if (!fail_step) fail_step = own(dalloc<int>(R));
+    }
+
+    // After a synchronisation: reports a resident launch whose parts lost
+    // each other (its results are not to be used).
+    void check_resident()
+    {
+        if (!res_err || *(volatile int*)res_err == 0) return;
+        *res_err = 0;
+        throw Failure{SNH_ERR_HIP, "resident steps: a wait for a neighbouring part timed out"};
     }
 
     void build(const snh_spec& sp)
@@ -602,14 +654,13 @@ struct SystemImpl final : snh_system {
         }
         SNH_REQUIRE(sp.layout == SNH_LAYOUT_AUTO || sp.layout == SNH_LAYOUT_GHOST, SNH_ERR_INVALID,
                     "layout must be SNH_LAYOUT_AUTO or SNH_LAYOUT_GHOST");
-        // one small :dipole replica without Ewald: midpoint steps in one
-        // cooperative launch (ghost layout), above the one-workgroup size
-        {
-            const long long sites = sp.nreplicas == 1 ? (long long)sp.dims[0] * sp.dims[1] * sp.dims[2] * na : 0;
-            coop = N == 0 && !ewald && R == 1 && sites > kPersist &&
-                   sites <= env_int("SNH_COOP_MAX_SITES", kCoopMaxSites) && env_int("SNH_COOP", 1) != 0;
-        }
-        if (N == 0 && sp.layout == SNH_LAYOUT_AUTO && !coop) {
+        // one small :dipole replica without Ewald, above the one-workgroup
+        // size: steps in one cooperative launch
+        const long long sites1 = sp.nreplicas == 1 ? (long long)sp.dims[0] * sp.dims[1] * sp.dims[2] * na : 0;
+        coop = N == 0 && !ewald && R == 1 && sites1 > kResOneWg &&
+               sites1 <= std::min(env_int("SNH_COOP_MAX_SITES", kResMaxSites), kResMaxSites) &&
+               env_int("SNH_COOP", 1) != 0;
+        if (N == 0 && sp.layout == SNH_LAYOUT_AUTO && !(coop && sites1 <= kResGhostSites)) {
             int dev = 0;
             SNH_HIP(hipGetDevice(&dev));
             hipDeviceProp_t prop;
@@ -878,15 +929,13 @@ struct SystemImpl final : snh_system {
         atol2 = own(dalloc<double>(R));
         nscale = own(dalloc<T>(R));
         SNH_HIP(hipHostMalloc((void**)&pinned, sizeof(double) * R, hipHostMallocDefault));
-        SNH_HIP(hipHostMalloc((void**)&pinned_i, sizeof(int) * R, hipHostMallocDefault));
+        SNH_HIP(hipHostMalloc((void**)&pinned_i, sizeof(int) * (R + 1), hipHostMallocDefault));
         if (ewald) build_ewald(sp);
         long long max_sites = 0;
         for (const auto& ri : reps) max_sites = std::max(max_sites, (long long)ri.ncell * na);
-        // measured crossover: faster up to one site per thread of the
-        // workgroup (64 sites: 5.8 vs 8.8 us per Langevin step), slower beyond
-        // (4096 sites: 64 vs 10.7 us)
         persist = N == 0 && !ewald && !tiled && env_int("SNH_PERSIST", 1) != 0 &&
-                  max_sites <= env_int("SNH_PERSIST_MAX_SITES", kPersist);
+                  max_sites <= std::min(env_int("SNH_PERSIST_MAX_SITES", kResOneWg), kResOneWg);
+        if (persist || coop) build_resident(bstart);
         mid_sync = env_int("SNH_MID_SYNC", 0) != 0;
         const int pair_env = env_int("SNH_PAIR", 1);
         if (tiled && !ewald && R >= 2 && pair_env != 0) {
@@ -1139,6 +1188,7 @@ struct SystemImpl final : snh_system {
         std::vector<T> h((size_t)np * total);
         SNH_HIP(hipMemcpyAsync(h.data(), P, sizeof(T) * h.size(), hipMemcpyDeviceToHost, st));
         SNH_HIP(hipStreamSynchronize(st));
+        check_resident();
         for_each_padded([&](uint32_t g, long long s, bool interior) {
             if (!interior) return;
             for (int p = 0; p < np; p++) x[(size_t)np * s + p] = (double)h[(size_t)p * total + g];
@@ -1829,17 +1879,26 @@ struct SystemImpl final : snh_system {
             if (!dz_valid) launch_sun_expected_spin<T>(C, nblocks, X, Dz, st);
             dz_valid = true;
         }
-        if (persist) {
+        if (persist || (coop && graph_steps == 0 && !timer.enabled &&
+                         nsteps >= res_min_steps(replica_sites(0)))) {
             // chunks bound the length of one launch
-            for (int s = 0; s < nsteps; s += 4096) {
+            bool done = true;
+            for (int s = 0; s < nsteps && done; s += 4096) {
                 nz.step = step0 + (uint64_t)s;
                 hipEvent_t e = tbegin();
-                launch_dipole_langevin_persist<T>(C, R, d_rblk, X, Xp, Xo, nz, tdt, tl, std::min(4096, nsteps - s),
-                                                  st);
-                tend("dipole_persist", e);
+                if (res_ex) launch_res_clear(res_ex, res_words(res, sizeof(T)), conv_iter, fail_step, R, st);
+                const hipError_t le = launch_res_langevin<T>(C, res, res_args, X, nz, tdt, tl,
+                                                             std::min(4096, nsteps - s), st);
+                tend("dipole_resident", e);
+                if (le == hipSuccess) continue;
+                // parts the device cannot keep resident: launched stages from
+                // now on (same layout, same results)
+                (void)hipGetLastError();
+                SNH_REQUIRE(s == 0 && coop, SNH_ERR_HIP, "resident Langevin launch failed");
+                coop = done = false;
             }
             SNH_HIP(hipGetLastError());
-            return;
+            if (done) return;
         }
         int s = 0;
         // the first step of a handle runs eagerly (it also sets kernel attributes)
@@ -1882,7 +1941,6 @@ struct SystemImpl final : snh_system {
         SNH_REQUIRE(std::isfinite(dt) && dt > 0, SNH_ERR_INVALID, "Select positive dt");
         SNH_REQUIRE(damping >= 0, SNH_ERR_INVALID, "Select nonnegative damping");
         SNH_REQUIRE(max_iters >= 1, SNH_ERR_INVALID, "max_iters must be at least 1");
-        ensure_midpoint_buffers();
         // atol = tol * sqrt(length(S)), length counting sites (Integrators.jl:383)
         std::vector<double> a2(R);
         for (int r = 0; r < R; r++) {
@@ -1892,77 +1950,37 @@ struct SystemImpl final : snh_system {
         SNH_HIP(hipMemcpyAsync(atol2, a2.data(), sizeof(double) * R, hipMemcpyHostToDevice, st));
         SNH_HIP(hipStreamSynchronize(st));
         const T tdt = (T)dt, tl = (T)damping;
-        if (coop && !tiled && nsteps > 0) {
-            // every step iterated to convergence in one cooperative launch
-            if (!fail_step) fail_step = own(dalloc<int>(R));
-            if (!coop_partial) coop_partial = own(dalloc<double>(2 * (size_t)nblocks));
-            if (!coop_bar) coop_bar = own(dalloc<unsigned>(3));
-            launch_fill_int(fail_step, R, -1, st);
-            launch_fill_int(conv_iter, R, 0, st);
-            launch_fill_int(reinterpret_cast<int*>(coop_bar), 3, 0, st);
-            const GridBar bar{coop_bar, coop_bar + 1, reinterpret_cast<int*>(coop_bar + 2), 1u << 22};
+        if ((persist || coop) && R == 1 && nsteps > 0) {
+            // every step iterated to convergence on the device; one host check per call
             hipEvent_t e = tbegin();
-            const hipError_t le = launch_dipole_midpoint_coop<T>(C, nblocks, X, B1, B2, Bh, Bh2, tdt, tl, atol2,
-                                                                 max_iters, nsteps, conv_iter, fail_step,
-                                                                 coop_partial, bar, st);
-            tend("midpoint_coop", e);
+            launch_res_clear(res_ex, res_words(res, sizeof(T)), conv_iter, fail_step, R, st);
+            const hipError_t le = launch_res_midpoint<T>(C, res, res_args, X, tdt, tl, atol2, max_iters, nsteps,
+                                                         conv_iter, fail_step, res_sdd, st);
+            tend("midpoint_resident", e);
             if (le != hipSuccess) {
-                // a grid the device cannot keep resident: launched sweeps
-                // from now on (same layout, same results)
+                // parts the device cannot keep resident: launched sweeps from
+                // now on (same layout, same results)
                 (void)hipGetLastError();
+                SNH_REQUIRE(coop, SNH_ERR_HIP, "resident midpoint launch failed");
                 coop = false;
-                step_midpoint(dt, damping, tol, max_iters, nsteps, iters);
+            } else {
+                SNH_HIP(hipMemcpyAsync(pinned_i, conv_iter, sizeof(int), hipMemcpyDeviceToHost, st));
+                SNH_HIP(hipMemcpyAsync(pinned_i + 1, fail_step, sizeof(int), hipMemcpyDeviceToHost, st));
+                SNH_HIP(hipStreamSynchronize(st));
+                check_resident();
+                if (iters) iters[0] = pinned_i[0];
+                last_iters = pinned_i[0];
+                if (pinned_i[1] >= 0) {
+                    char msg[256];
+                    snprintf(msg, sizeof msg,
+                             "Spherical midpoint method failed to converge to tolerance %g after %d iterations.", tol,
+                             max_iters);
+                    throw Failure{SNH_ERR_NOCONVERGE, msg};
+                }
                 return;
             }
-            SNH_HIP(hipGetLastError());
-            int h[3];
-            SNH_HIP(hipMemcpyAsync(pinned_i, conv_iter, sizeof(int), hipMemcpyDeviceToHost, st));
-            SNH_HIP(hipStreamSynchronize(st));
-            h[0] = pinned_i[0];
-            SNH_HIP(hipMemcpyAsync(pinned_i, fail_step, sizeof(int), hipMemcpyDeviceToHost, st));
-            SNH_HIP(hipStreamSynchronize(st));
-            h[1] = pinned_i[0];
-            SNH_HIP(hipMemcpyAsync(pinned_i, coop_bar + 2, sizeof(int), hipMemcpyDeviceToHost, st));
-            SNH_HIP(hipStreamSynchronize(st));
-            h[2] = pinned_i[0];
-            SNH_REQUIRE(h[2] == 0, SNH_ERR_HIP, "cooperative midpoint: a grid barrier wait timed out");
-            if (iters) iters[0] = h[0];
-            last_iters = h[0];
-            if (h[1] >= 0) {
-                char msg[256];
-                snprintf(msg, sizeof msg,
-                         "Spherical midpoint method failed to converge to tolerance %g after %d iterations.", tol,
-                         max_iters);
-                throw Failure{SNH_ERR_NOCONVERGE, msg};
-            }
-            return;
         }
-        if (persist && R == 1 && nsteps > 0) {
-            // every step iterated to convergence on the device; one host check per call
-            if (!fail_step) fail_step = own(dalloc<int>(R));
-            launch_fill_int(fail_step, R, -1, st);
-            launch_fill_int(conv_iter, R, 0, st);
-            hipEvent_t e = tbegin();
-            launch_dipole_midpoint_persist<T>(C, R, d_rblk, X, B1, B2, Bh, Bh2, tdt, tl, atol2, max_iters, nsteps,
-                                              conv_iter, fail_step, st);
-            tend("midpoint_persist", e);
-            SNH_HIP(hipGetLastError());
-            SNH_HIP(hipMemcpyAsync(pinned_i, conv_iter, sizeof(int) * R, hipMemcpyDeviceToHost, st));
-            SNH_HIP(hipStreamSynchronize(st));
-            const int its = pinned_i[0];
-            SNH_HIP(hipMemcpyAsync(pinned_i, fail_step, sizeof(int) * R, hipMemcpyDeviceToHost, st));
-            SNH_HIP(hipStreamSynchronize(st));
-            if (iters) iters[0] = its;
-            last_iters = its;
-            if (pinned_i[0] >= 0) {
-                char msg[256];
-                snprintf(msg, sizeof msg,
-                         "Spherical midpoint method failed to converge to tolerance %g after %d iterations.", tol,
-                         max_iters);
-                throw Failure{SNH_ERR_NOCONVERGE, msg};
-            }
-            return;
-        }
+        ensure_midpoint_buffers();
         // Groups of steps run optimistically: each step gets a fixed budget of
         // iterations (the last count + 1; iterations after convergence are
         // no-ops) and no host check; a group in which some replica needs more
@@ -2141,8 +2159,12 @@ struct SystemImpl final : snh_system {
     // converged iteration and its iteration count.
     T* midpoint_one(double dt, double tol, int max_iters, int* it_out)
     {
+        ensure_midpoint_buffers();
+        res_sdd = B1;  // a resident launch writes S'' there
         step_midpoint(dt, 0.0, tol, max_iters, 1, it_out);
-        return (*it_out % 2 == 1) ? B1 : B2;  // S'' of iteration m lives in B1 for odd m, B2 for even m
+        res_sdd = nullptr;
+        // launched sweeps: S'' of iteration m lives in B1 for odd m, B2 for even m
+        return persist || coop || *it_out % 2 == 1 ? B1 : B2;
     }
 
     void midpoint_record(double dt, double tol, int max_iters, int nsteps, int every) override
@@ -2370,6 +2392,7 @@ struct SystemImpl final : snh_system {
         energy_launch(partial, d_out, true);
         SNH_HIP(hipMemcpyAsync(pinned, d_out, sizeof(double) * R, hipMemcpyDeviceToHost, st));
         SNH_HIP(hipStreamSynchronize(st));
+        check_resident();
         for (int r = 0; r < R; r++) E[r] = pinned[r];
     }
 
@@ -2407,7 +2430,11 @@ struct SystemImpl final : snh_system {
         download_planes(Xp, planes, out);
     }
 
-    void synchronize() override { SNH_HIP(hipStreamSynchronize(st)); }
+    void synchronize() override
+    {
+        SNH_HIP(hipStreamSynchronize(st));
+        check_resident();
+    }
 
     void enable_timing(bool on) override
     {

@@ -199,214 +199,6 @@ __global__ __launch_bounds__(kBlock) void k_dipole_mid_finalize_mu(Couplings<T> 
                       normalize_dipole(V3<T>{(s.x + s.x) / 2, (s.y + s.y) / 2, (s.z + s.z) / 2}, kap));
 }
 
-// ---------------------------------------------------------------------------
-// Persistent kernels for small replicas: one workgroup of kPersist threads
-// per replica runs many steps, its 256-site blocks kPersistLanes at a time,
-// with workgroup barriers between stages instead of kernel launches (and,
-// for the midpoint, instead of a host convergence check per step).  A
-// workgroup runs on one CU, and __syncthreads orders global memory at
-// workgroup scope, so one stage's stores are visible to the next.
-
-template <typename T, typename F>
-__device__ __forceinline__ void for_replica_sites(const Couplings<T>& C, int b0, int b1, F f)
-{
-    const int sub = (int)threadIdx.x / kBlock, lane = (int)threadIdx.x % kBlock;
-    for (int b = b0 + sub; b < b1; b += kPersistLanes) {
-        const SiteCoord sc = site_coord_at(C.blocks, C.reps, C.G, b, lane);
-        if (sc.valid) f(sc);
-    }
-}
-
-// Sum over the workgroup, returned to every thread (two barriers).
-__device__ __forceinline__ double persist_sum(double v, double* red)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double t = 0;
-#pragma unroll
-    for (int k = 0; k < kPersist / 64; k++) t += red[k];
-    __syncthreads();
-    return t;
-}
-
-// nsteps Heun steps of replica blockIdx.x (steps nz.step, nz.step + 1, ...).
-template <typename T, int CH, bool kIso>
-__global__ __launch_bounds__(kPersist) void k_dipole_langevin_persist(Couplings<T> C, const int* __restrict__ rblk,
-                                                                      T* X, T* Xp, T* Xo, NoiseArgs<T> nz, T dt,
-                                                                      T lambda, int nsteps)
-{
-    const int b0 = rblk[blockIdx.x], b1 = rblk[blockIdx.x + 1];
-    const unsigned long long step0 = nz.step;
-    for (int s = 0; s < nsteps; s++) {
-        nz.step = step0 + (unsigned long long)s;
-        for_replica_sites(C, b0, b1, [&](const SiteCoord& sc) __attribute__((always_inline)) {
-            dipole_predict_site<T, CH, kIso>(C, sc, X, Xp, Xo, nullptr, nz, dt, lambda);
-        });
-        __syncthreads();
-        for_replica_sites(C, b0, b1, [&](const SiteCoord& sc) __attribute__((always_inline)) {
-            dipole_correct_site<T, CH, kIso>(C, sc, Xp, Xo, X, nullptr, dt, lambda);
-        });
-        __syncthreads();
-    }
-}
-
-// nsteps spherical-midpoint steps of replica r = blockIdx.x, each iterated
-// to fast_isapprox convergence on the device: Shat of iteration m lives in
-// hats[m % 2] (hats = {Bh2, Bh}), S'' in bufs[m % 2] (bufs = {B2, B1}).
-// iters_out[r]: iterations of the last step; a step that does not converge
-// within max_iters sets fail_step[r] and leaves X at the previous step.
-template <typename T, int CH>
-__global__ __launch_bounds__(kPersist) void k_dipole_midpoint_persist(Couplings<T> C, const int* __restrict__ rblk,
-                                                                      T* X, T* B1, T* B2, T* Bh, T* Bh2, T dt,
-                                                                      T lambda, const double* __restrict__ atol2,
-                                                                      int max_iters, int nsteps,
-                                                                      int* __restrict__ iters_out,
-                                                                      int* __restrict__ fail_step)
-{
-    __shared__ double red[kPersist / 64];
-    const int r = blockIdx.x;
-    const int b0 = rblk[r], b1 = rblk[r + 1];
-    T* const bufs[2] = {B2, B1};
-    T* const hats[2] = {Bh2, Bh};
-    const double a2 = atol2[r];
-    for (int s = 0; s < nsteps; s++) {
-        // the first guess S' = S: Shat = kappa n((S + S)/2) = kappa n(S)
-        for_replica_sites(C, b0, b1, [&](const SiteCoord& sc) __attribute__((always_inline)) {
-            store3_images(Bh, C.total, sc, C.G, normalize_dipole(planes(X, C.total)(sc.g), ldc(C.kappa, sc.i)));
-        });
-        __syncthreads();
-        int it = 0;
-        bool conv = false;
-        while (!conv && it < max_iters) {
-            ++it;
-            const T* S1 = it == 1 ? X : bufs[(it + 1) % 2];
-            T* S2 = bufs[it % 2];
-            const T* hat = hats[it % 2];
-            T* hat_next = hats[(it + 1) % 2];
-            double d2 = 0;
-            for_replica_sites(C, b0, b1, [&](const SiteCoord& sc) __attribute__((always_inline)) {
-                d2 += dipole_mid_sweep_site<T, CH>(C, sc, X, S1, S2, hat, nullptr, dt, lambda, hat_next);
-            });
-            const double t = persist_sum(d2, red);  // uniform: every thread sums the same partials
-            conv = t <= a2 && !isnan(t);
-        }
-        if (!conv) {
-            if (threadIdx.x == 0) {
-                fail_step[r] = s;
-                iters_out[r] = it;
-            }
-            return;
-        }
-        const T* S2 = bufs[it % 2];
-        for_replica_sites(C, b0, b1, [&](const SiteCoord& sc) __attribute__((always_inline)) {
-            store3_images(X, C.total, sc, C.G, normalize_dipole(planes(S2, C.total)(sc.g), ldc(C.kappa, sc.i)));
-        });
-        __syncthreads();
-        if (threadIdx.x == 0) iters_out[r] = it;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Cooperative midpoint for one small replica: one workgroup per 256-site
-// block, all resident (cooperative launch), a grid barrier per fixed-point
-// iteration instead of a sweep launch and a check launch.
-
-// Barrier over the gridDim.x workgroups of a cooperative launch: a counter
-// and a generation in device memory (zero at launch).  Thread 0 of each
-// workgroup arrives after a release fence at agent scope (its workgroup's
-// stores become visible device-wide) and waits for the generation to move
-// with acquire loads; the last to arrive resets the counter and moves it.
-// A wait longer than bar.spin polls sets *bar.err and proceeds, and once
-// *bar.err is set no wait lasts, so every wave still exits promptly.
-__device__ __forceinline__ void grid_sync(const GridBar& bar, unsigned& epoch)
-{
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        const unsigned arrived = __hip_atomic_fetch_add(bar.count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (arrived == gridDim.x - 1) {
-            __hip_atomic_store(bar.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(bar.gen, epoch + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            unsigned n = 0;
-            while (__hip_atomic_load(bar.gen, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) == epoch) {
-                if (++n > bar.spin || __hip_atomic_load(bar.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                    __hip_atomic_store(bar.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    }
-    ++epoch;
-    __syncthreads();
-}
-
-// nsteps spherical-midpoint steps of the handle's one replica, each iterated
-// to fast_isapprox convergence as k_dipole_midpoint_persist does, workgroup
-// b sweeping block b.  The residual of iteration m: each workgroup's block
-// sum goes to partial[(m % 2) nb + b] and, after the barrier, every
-// workgroup sums the nb partials as k_midpoint_check does, so all take the
-// same decision (the same one the launched sweeps take).
-template <typename T, int CH>
-__global__ __launch_bounds__(kBlock) void k_dipole_midpoint_coop(Couplings<T> C, T* X, T* B1, T* B2, T* Bh, T* Bh2,
-                                                                 T dt, T lambda, const double* __restrict__ atol2,
-                                                                 int max_iters, int nsteps,
-                                                                 int* __restrict__ iters_out,
-                                                                 int* __restrict__ fail_step, double* partial,
-                                                                 GridBar bar)
-{
-    __shared__ double s_tot;
-    const int nb = (int)gridDim.x;
-    unsigned epoch = 0;
-    const SiteCoord sc = site_coord(C.blocks, C.reps, C.G);
-    T* const bufs[2] = {B2, B1};
-    T* const hats[2] = {Bh2, Bh};
-    const double a2 = atol2[0];
-    for (int s = 0; s < nsteps; s++) {
-        // the first guess S' = S: Shat = kappa n((S + S)/2) = kappa n(S)
-        if (sc.valid)
-            store3_images(Bh, C.total, sc, C.G, normalize_dipole(planes(X, C.total)(sc.g), ldc(C.kappa, sc.i)));
-        grid_sync(bar, epoch);
-        int it = 0;
-        bool conv = false;
-        while (!conv && it < max_iters) {
-            ++it;
-            const T* S1 = it == 1 ? X : bufs[(it + 1) % 2];
-            double d2 = 0;
-            if (sc.valid)
-                d2 = dipole_mid_sweep_site<T, CH>(C, sc, X, S1, bufs[it % 2], hats[it % 2], nullptr, dt, lambda,
-                                                  hats[(it + 1) % 2]);
-            // slots alternate: a workgroup rewrites slot it % 2 only after the
-            // next barrier, by which every workgroup has read it
-            double* part = partial + (it % 2) * nb;
-            const double t = block_sum(d2);
-            if (threadIdx.x == 0) part[blockIdx.x] = t;
-            grid_sync(bar, epoch);
-            double v = 0;
-            for (int k = (int)threadIdx.x; k < nb; k += kBlock) v += part[k];
-            const double tot = block_sum(v);
-            if (threadIdx.x == 0) s_tot = tot;
-            __syncthreads();
-            conv = s_tot <= a2 && !isnan(s_tot);  // uniform over the grid
-        }
-        if (!conv) {
-            if (blockIdx.x == 0 && threadIdx.x == 0) {
-                fail_step[0] = s;
-                iters_out[0] = it;
-            }
-            return;
-        }
-        if (sc.valid)
-            store3_images(X, C.total, sc, C.G,
-                          normalize_dipole(planes(bufs[it % 2], C.total)(sc.g), ldc(C.kappa, sc.i)));
-        if (blockIdx.x == 0 && threadIdx.x == 0) iters_out[0] = it;
-    }
-}
-
 template <typename T, int CH>
 __global__ __launch_bounds__(kBlock) void k_dipole_grad(Couplings<T> C, const T* __restrict__ S,
                                                         const T* __restrict__ phi, T* __restrict__ dE)
@@ -658,47 +450,6 @@ void launch_step_advance(unsigned long long* p, hipStream_t st)
     hipLaunchKernelGGL(k_step_advance, dim3(1), dim3(64), 0, st, p);
 }
 
-template <typename T>
-void launch_dipole_langevin_persist(const Couplings<T>& C, int R, const int* rblk, T* X, T* Xp, T* Xo,
-                                   const NoiseArgs<T>& nz, T dt, T lambda, int nsteps, hipStream_t st)
-{
-#define SNH_LP(CH, ISO)                                                                                      \
-    hipLaunchKernelGGL((k_dipole_langevin_persist<T, CH, ISO>), dim3(R), dim3(kPersist), 0, st, C, rblk, X, Xp, \
-                       Xo, nz, dt, lambda, nsteps)
-    if (C.chunk == 18) {
-        if (C.iso) SNH_LP(18, true); else SNH_LP(18, false);
-    } else if (C.chunk == 9) {
-        if (C.iso) SNH_LP(9, true); else SNH_LP(9, false);
-    } else {
-        if (C.iso) SNH_LP(6, true); else SNH_LP(6, false);
-    }
-#undef SNH_LP
-}
-
-template <typename T>
-void launch_dipole_midpoint_persist(const Couplings<T>& C, int R, const int* rblk, T* X, T* B1, T* B2, T* Bh, T* Bh2,
-                                    T dt, T lambda, const double* atol2, int max_iters, int nsteps, int* iters_out,
-                                    int* fail_step, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_dipole_midpoint_persist<T, 6>), dim3(R), dim3(kPersist), 0, st, C, rblk, X, B1, B2, Bh,
-                       Bh2, dt, lambda, atol2, max_iters, nsteps, iters_out, fail_step);
-}
-
-template <typename T>
-hipError_t launch_dipole_midpoint_coop(const Couplings<T>& C, int nblocks, T* X, T* B1, T* B2, T* Bh, T* Bh2, T dt,
-                                       T lambda, const double* atol2, int max_iters, int nsteps, int* iters_out,
-                                       int* fail_step, double* partial, const GridBar& bar, hipStream_t st)
-{
-    Couplings<T> c = C;
-    GridBar b = bar;
-    void* args[] = {&c, &X, &B1, &B2, &Bh, &Bh2, &dt, &lambda, &atol2, &max_iters, &nsteps, &iters_out, &fail_step,
-                    &partial, &b};
-    const void* fn = C.chunk == 18   ? reinterpret_cast<const void*>(&k_dipole_midpoint_coop<T, 18>)
-                     : C.chunk == 9 ? reinterpret_cast<const void*>(&k_dipole_midpoint_coop<T, 9>)
-                                    : reinterpret_cast<const void*>(&k_dipole_midpoint_coop<T, 6>);
-    return hipLaunchCooperativeKernel(fn, dim3(nblocks), dim3(kBlock), args, 0, st);
-}
-
 #define SNH_INST(T)                                                                                              \
     template void launch_dipole_predict<T>(const Couplings<T>&, int, const T*, T*, T*, const T*,                \
                                            const NoiseArgs<T>&, T, T, hipStream_t);                             \
@@ -706,9 +457,6 @@ hipError_t launch_dipole_midpoint_coop(const Couplings<T>& C, int nblocks, T* X,
                                            hipStream_t);                                                         \
     template void launch_dipole_midpoint_hat<T>(const Couplings<T>&, int, const T*, const T*, T*, const int*,    \
                                                 hipStream_t);                                                    \
-    template hipError_t launch_dipole_midpoint_coop<T>(const Couplings<T>&, int, T*, T*, T*, T*, T*, T, T,       \
-                                                       const double*, int, int, int*, int*, double*,             \
-                                                       const GridBar&, hipStream_t);                             \
     template void launch_dipole_midpoint_iter<T>(const Couplings<T>&, int, const T*, const T*, T*, const T*,     \
                                                  const T*, T, T, double*, const int*, T*, hipStream_t);                     \
     template void launch_dipole_midpoint_finalize_mu<T>(const Couplings<T>&, int, T*, const T*, const T*,        \
@@ -716,10 +464,6 @@ hipError_t launch_dipole_midpoint_coop(const Couplings<T>& C, int nblocks, T* X,
     template void launch_dipole_midpoint_finalize<T>(const Couplings<T>&, int, T*, const T*, const T*,           \
                                                      const int*, int, T*, hipStream_t);                              \
     template void launch_dipole_grad<T>(const Couplings<T>&, int, const T*, const T*, T*, hipStream_t);          \
-    template void launch_dipole_langevin_persist<T>(const Couplings<T>&, int, const int*, T*, T*, T*,             \
-                                                    const NoiseArgs<T>&, T, T, int, hipStream_t);                \
-    template void launch_dipole_midpoint_persist<T>(const Couplings<T>&, int, const int*, T*, T*, T*, T*, T*, T, \
-                                                    T, const double*, int, int, int*, int*, hipStream_t);        \
     template void launch_dipole_energy<T>(const Couplings<T>&, int, const T*, const T*, double*, hipStream_t);
 
 SNH_INST(float)

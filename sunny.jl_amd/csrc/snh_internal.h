@@ -2,7 +2,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <string>
+#include <vector>
 
 #include "../../include/sunny_hip.h"
 #include "snh_device.h"
@@ -194,34 +196,72 @@ void launch_fill_int(int* p, int n, int v, hipStream_t st);
 // max_iter[r]: largest iteration count of the group's steps 0..s; last_it[r]:
 // step s's count; conv_iter cleared for the next step.
 void launch_mid_budget(int* conv_iter, int* fail_step, int* max_iter, int* last_it, int R, int s, hipStream_t st);
-// Persistent small-replica kernels (one workgroup per replica, rblk: its
-// range of logical blocks): nsteps Langevin steps, or nsteps midpoint steps
-// iterated to convergence on the device (iters_out / fail_step per replica).
-template <typename T>
-void launch_dipole_langevin_persist(const Couplings<T>& C, int R, const int* rblk, T* X, T* Xp, T* Xo,
-                                   const NoiseArgs<T>& nz, T dt, T lambda, int nsteps, hipStream_t st);
-// Largest one-replica handle stepped by the cooperative midpoint launch.
-constexpr int kCoopMaxSites = 8192;
-// Barrier state of a cooperative launch: count and gen zero at launch;
-// *err set when a wait exceeded spin polls.
-struct GridBar {
-    unsigned* count;
-    unsigned* gen;
-    int* err;
-    unsigned spin;
+// Small :dipole replicas (either layout, no Ewald) stepped inside one launch
+// per call (snh_resident.hip).  Replicas of up to kResOneWg sites are one
+// workgroup; a larger one, up to kResMaxSites sites, is cut into parts of at
+// most 64 sites, one workgroup of kResThreads each, that exchange their
+// border sites.  Measured against the launch per stage, us per Langevin step
+// of 200 and per midpoint step of 20 (FP64, tol 1e-12): cubic 16^3 4.3 / 11.2
+// and 35 / 84; cubic 28^3 (21,952 sites) 5.6 / 11.2 and 69 / 84; pyrochlore
+// 12^3 x 16 (27,648) 12.1 / 14.3 and 90 / 123; cubic 32^3 (32,768) 8.3 / 11.1
+// but 93 / 84: hence the bound.
+constexpr int kResOneWg = 512;
+constexpr int kResThreads = 256;
+constexpr int kResMaxSites = 28672;
+constexpr int kResGhostSites = 8192;  // up to here AUTO takes the ghost layout
+// Langevin steps of a call from which parts pay (a cooperative launch costs
+// about 20 us more than a plain one): calls of 4 steps 17.1 against 17.7 us a
+// step at 4096 sites, 20.1 / 20.4 at 8192, but 18.2 / 17.7 at 21,952 and 24.9 /
+// 20.6 at 27,648; calls of 8 steps 10.6 / 14.3, 14.1 / 17.0, 12.0 / 14.4, 18.5 / 18.2.
+constexpr int res_min_steps(long long sites) { return 4 + (int)(sites / 8192); }
+struct ResWg {
+    int r;                  // replica
+    int first;              // the replica's first part (reports iterations)
+    int nlane, lane0;       // lanes with sites (a multiple of 64) and their entries in `lane`
+    int laner;              // entries of the replica's first part
+    int nhalo, halo0;       // halo sites and their entries in `halo`
+    int nbr0;               // LDS indices [nslot][nlane] in `nbr`
+    int ex0, exr;           // exchange position of lane 0, and of the replica's first lane
+    int res0, resr, nresr;  // residual words: this part's first, the replica's first and count (0: one part)
 };
-// nsteps midpoint steps of a one-replica handle (ghost layout, no Ewald) in
-// one cooperative launch of nblocks workgroups (one per block); partial:
-// [2 nblocks].  Returns the launch status (a grid that cannot be resident is
-// refused).
+struct ResPlan {
+    std::vector<ResWg> wg;
+    std::vector<int> lane;  // cell * na + sublattice of every lane, -1: idle
+    std::vector<int> halo;  // exchange positions, relative to exr
+    std::vector<unsigned short> nbr;
+    int nslot = 0, nex = 0, nres = 0, threads = 0;
+    bool uni = false;       // one sublattice
+    bool shared = false;    // some replica spans several workgroups
+    size_t lds = 0;
+};
+struct ResArgs {
+    const ResWg* wg;
+    const int* lane;
+    const int* halo;
+    const unsigned short* nbr;
+    unsigned long long* ex;   // [2][words of a site][nex] exchanged sites
+    unsigned long long* res;  // [2][2][nres] residuals
+    int nslot, nex, nres;
+    unsigned spin;            // polls after which a wait is given up
+    int* err;                 // set then (host memory)
+};
+// The plan of all replicas, or false where there is none: a replica of more
+// than kResMaxSites sites, a part whose spins do not fit lds_max bytes, a
+// bond without its reverse.  slots: cell offset and target sublattice of
+// every padded gather slot; bstart: slot ranges of the sublattices.
+bool plan_resident(int na, const std::vector<std::array<int, 3>>& dims, const std::vector<int>& bstart,
+                   const std::vector<std::array<int, 4>>& slots, size_t elem, size_t lds_max, ResPlan& out);
+size_t res_words(const ResPlan& P, size_t elem);  // 8-byte words of ex and res together
+void launch_res_clear(unsigned long long* words, size_t n, int* iters, int* fail, int R, hipStream_t st);
+// Both return the launch status (parts that cannot all be resident are
+// refused).  Sdd (may be null): receives S'' of the last iteration.
 template <typename T>
-hipError_t launch_dipole_midpoint_coop(const Couplings<T>& C, int nblocks, T* X, T* B1, T* B2, T* Bh, T* Bh2, T dt,
-                                       T lambda, const double* atol2, int max_iters, int nsteps, int* iters_out,
-                                       int* fail_step, double* partial, const GridBar& bar, hipStream_t st);
+hipError_t launch_res_langevin(const Couplings<T>& C, const ResPlan& P, const ResArgs& A, T* X,
+                               const NoiseArgs<T>& nz, T dt, T lambda, int nsteps, hipStream_t st);
 template <typename T>
-void launch_dipole_midpoint_persist(const Couplings<T>& C, int R, const int* rblk, T* X, T* B1, T* B2, T* Bh, T* Bh2,
-                                    T dt, T lambda, const double* atol2, int max_iters, int nsteps, int* iters_out,
-                                    int* fail_step, hipStream_t st);
+hipError_t launch_res_midpoint(const Couplings<T>& C, const ResPlan& P, const ResArgs& A, T* X, T dt, T lambda,
+                               const double* atol2, int max_iters, int nsteps, int* iters_out, int* fail_step,
+                               T* Sdd, hipStream_t st);
 
 // Sampled correlations (snh_corr.hip): buffers are FP64 complex (re, im).
 template <typename T>

@@ -22,6 +22,19 @@ __device__ __forceinline__ V3<T> cross3(V3<T> a, V3<T> b)
     return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
 
+// |s|^2 with its two fused multiply-adds spelled out: which product of a sum
+// of squares the compiler would fuse differs from kernel to kernel, and the
+// launched and the resident steps agree bitwise.
+__device__ __forceinline__ double norm2(V3<double> s)
+{
+    return __builtin_fma(s.z, s.z, __builtin_fma(s.y, s.y, s.x * s.x));
+}
+
+__device__ __forceinline__ float norm2(V3<float> s)
+{
+    return __builtin_fmaf(s.z, s.z, __builtin_fmaf(s.y, s.y, s.x * s.x));
+}
+
 // kappa * s/|s| (normalize_dipole, System.jl:421-423).  FP64 state:
 // correctly rounded sqrt and divide.  FP32 state: FP32 throughout, with the
 // hardware reciprocal square root (v_rsq_f32, 1 ulp): |result| is within
@@ -29,14 +42,14 @@ __device__ __forceinline__ V3<T> cross3(V3<T> a, V3<T> b)
 __device__ __forceinline__ V3<double> normalize_dipole(V3<double> s, double kappa)
 {
     if (kappa == 0.0) return {0, 0, 0};
-    const double f = kappa / sqrt(s.x * s.x + s.y * s.y + s.z * s.z);
+    const double f = kappa / sqrt(norm2(s));
     return {s.x * f, s.y * f, s.z * f};
 }
 
 __device__ __forceinline__ V3<float> normalize_dipole(V3<float> s, float kappa)
 {
     if (kappa == 0.0f) return {0, 0, 0};
-    const float f = kappa * __builtin_amdgcn_rsqf(s.x * s.x + s.y * s.y + s.z * s.z);
+    const float f = kappa * __builtin_amdgcn_rsqf(norm2(s));
     return {s.x * f, s.y * f, s.z * f};
 }
 
@@ -49,7 +62,7 @@ __device__ __forceinline__ V3<double> normalize_dipole_mu(V3<double> s, double k
         mu = 0;
         return {0, 0, 0};
     }
-    const double n = sqrt(s.x * s.x + s.y * s.y + s.z * s.z);
+    const double n = sqrt(norm2(s));
     const double f = kappa / n;
     mu = n / kappa;
     return {s.x * f, s.y * f, s.z * f};
@@ -61,7 +74,7 @@ __device__ __forceinline__ V3<float> normalize_dipole_mu(V3<float> s, float kapp
         mu = 0;
         return {0, 0, 0};
     }
-    const float f = kappa * __builtin_amdgcn_rsqf(s.x * s.x + s.y * s.y + s.z * s.z);
+    const float f = kappa * __builtin_amdgcn_rsqf(norm2(s));
     mu = __builtin_amdgcn_rcpf(f);
     return {s.x * f, s.y * f, s.z * f};
 }

@@ -1,0 +1,99 @@
+"""Small :dipole replicas stepped inside one launch per call, against the
+launch per stage on the same layout: sizes around one workgroup and around
+the largest exchange, ragged parts, axes shorter than a bond, many
+sublattices, and every kind of bond and onsite term.
+
+Both run the same per-site arithmetic.  Seven Langevin or midpoint steps
+round about 7 x 20 times; with the spread of one rounding over the steps
+(at most tenfold) that is 7 x 20 x 10 x 2^-53 = 1.6e-13 in FP64 and 8e-5 in
+FP32, relative to |S|.
+"""
+import numpy as np
+import pytest
+
+import sunnyhip as sh
+
+from helpers import announce, rel_err
+
+pytestmark = pytest.mark.gpu
+
+TOL = {64: 1.6e-13, 32: 8e-5}
+
+
+def general_model(dims, precision):
+    """Anisotropic exchange, biquadratic bonds, a field, Stevens terms to order 6."""
+    s = sh.System(sh.cubic_crystal(1.0), [(0, sh.Moment(s=3, g=2))], "dipole", dims=dims, seed=5, precision=precision)
+    J = np.array([[1.0, 0.2, -0.1], [0.1, 0.8, 0.05], [0.0, -0.2, 1.1]])
+    sh.set_exchange_(s, J, sh.Bond(0, 0, (1, 0, 0)))
+    sh.set_exchange_(s, 0.5, sh.Bond(0, 0, (0, 1, 0)), biquad=0.03,
+                     propagate=[sh.Bond(0, 0, (0, 1, 0)), sh.Bond(0, 0, (0, 0, 1))])
+    sh.set_onsite_coupling_(s, lambda S: 0.02 * S[2] @ S[2] @ S[2] @ S[2] +
+                            0.001 * S[0] @ S[0] @ S[0] @ S[0] @ S[0] @ S[0], 0)
+    sh.set_field_(s, [0.3, -0.1, 0.2])
+    sh.randomize_spins_(s)
+    return s
+
+
+def inhomogeneous(dims, precision):
+    """One sublattice per site (a vacancy among them): parts of a single cell."""
+    s = sh.to_inhomogeneous(sh.workloads.cubic_model(dims=dims, seed=6, precision=precision))
+    sh.set_vacancy_at_(s, (1, 0, 1, 0))
+    return s
+
+
+def build(kind, dims, precision):
+    if kind == "cubic":
+        return sh.workloads.cubic_model(dims=dims, seed=4, precision=precision)
+    if kind == "pyrochlore":
+        return sh.workloads.pyrochlore_model(dims=dims, seed=4, precision=precision)
+    return {"general": general_model, "inhomogeneous": inhomogeneous}[kind](dims, precision)
+
+
+@pytest.mark.parametrize("kind,dims,precision,layout", [
+    ("cubic", (1, 1, 1), 64, 1),       # one site, bonded to itself
+    ("cubic", (8, 8, 8), 64, 1),       # 512 sites: the largest single workgroup
+    ("cubic", (27, 19, 1), 64, 1),     # 513 sites: the smallest that is cut
+    ("cubic", (2, 1, 300), 64, 1),     # axes shorter than the parts
+    ("cubic", (19, 17, 13), 32, 1),    # ragged parts
+    ("cubic", (20, 20, 20), 64, 1),    # 125 parts
+    ("cubic", (16, 16, 32), 32, 1),
+    ("cubic", (28, 32, 32), 64, 1),    # 28672 sites: the most
+    ("cubic", (27, 29, 31), 32, 0),    # tiled layout
+    ("pyrochlore", (12, 11, 12), 32, 0),
+    ("pyrochlore", (2, 3, 5), 64, 1),  # one workgroup, sixteen sublattices
+    ("pyrochlore", (5, 3, 4), 64, 1),  # four cells a part
+    ("pyrochlore", (8, 8, 8), 32, 1),
+    ("general", (5, 6, 7), 64, 1),
+    ("general", (11, 9, 8), 64, 1),
+    ("general", (11, 9, 8), 32, 1),
+    ("inhomogeneous", (9, 9, 9), 64, 1),
+])
+def test_resident_steps_match_launches(kind, dims, precision, layout, monkeypatch):
+    announce(f"resident vs launched {kind} {dims} fp{precision} layout {layout}")
+
+    def handle(on):
+        monkeypatch.setenv("SNH_PERSIST", on)
+        monkeypatch.setenv("SNH_COOP", on)
+        s = build(kind, dims, precision)
+        s.layout = layout
+        h = s._device()
+        assert h.query("layout") == layout
+        assert h.query("persistent") + h.query("cooperative") == int(on)
+        return s
+
+    a, b = handle("1"), handle("0")
+    kap = float(np.max(a.kappas))
+    lang = sh.Langevin(0.02 / kap, damping=0.1, kT=0.4)
+    sh.step_(a, lang, nsteps=7)
+    sh.step_(b, lang, nsteps=7)
+    assert np.all(np.isfinite(b.dipoles_flat()))
+    assert rel_err(a.dipoles_flat(), b.dipoles_flat(), scale=kap) <= TOL[precision]
+    # the noise goes on where the call before ended
+    sh.step_(a, lang, nsteps=5)
+    sh.step_(b, lang, nsteps=5)
+    assert rel_err(a.dipoles_flat(), b.dipoles_flat(), scale=kap) <= 2 * TOL[precision]
+    b.set_state_flat(dip=a.dipoles_flat())
+    mid = sh.ImplicitMidpoint(0.01 / kap, damping=0.05, tol=1e-12 if precision == 64 else 1e-5)
+    ia, ib = sh.step_(a, mid, nsteps=7), sh.step_(b, mid, nsteps=7)
+    assert abs(int(ia[0]) - int(ib[0])) <= 1
+    assert rel_err(a.dipoles_flat(), b.dipoles_flat(), scale=kap) <= TOL[precision] + mid.tol
