@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "snh_internal.h"
+#include "snh_state.h"
 
 using namespace snh;
 
@@ -439,6 +440,26 @@ struct SystemImpl final : snh_system {
     std::vector<void*> owned;
     Couplings<T> C{};
     int* d_rblk = nullptr;
+    long long* d_rsite = nullptr;  // [R+1] first host site of every replica
+    // chunks of state transfers, two in turn (grown to kChunkBytes at most)
+    static constexpr size_t kChunkBytes = 4u << 20;
+    struct Transfer {
+        void* dev[2] = {nullptr, nullptr};
+        void* pin[2] = {nullptr, nullptr};
+        hipEvent_t ev[2] = {nullptr, nullptr};
+        size_t bytes = 0;
+        void release()
+        {
+            for (int k = 0; k < 2; k++) {
+                if (dev[k]) (void)hipFree(dev[k]);
+                if (pin[k]) (void)hipHostFree(pin[k]);
+                if (ev[k]) (void)hipEventDestroy(ev[k]);
+                dev[k] = pin[k] = nullptr;
+                ev[k] = nullptr;
+            }
+            bytes = 0;
+        }
+    } xfer;
     // state
     T* X = nullptr;     // current state (3 or 2N planes)
     T* Xp = nullptr;    // Heun stage S' (with ghosts)
@@ -576,6 +597,7 @@ struct SystemImpl final : snh_system {
         if (pinned) (void)hipHostFree(pinned);
         if (pinned_i) (void)hipHostFree(pinned_i);
         if (res_err) (void)hipHostFree(res_err);
+        xfer.release();
         if (st) (void)hipStreamDestroy(st);
     }
 
@@ -909,6 +931,9 @@ struct SystemImpl final : snh_system {
         C.total = total;
         C.G = G;
         d_rblk = own(dupload(rblk));
+        std::vector<long long> rsite(R + 1, 0);
+        for (int r = 0; r < R; r++) rsite[r + 1] = rsite[r] + (long long)reps[r].ncell * na;
+        d_rsite = own(dupload(rsite));
 
         X = own(dalloc<T>((size_t)planes * total));
         Xp = own(dalloc<T>((size_t)planes * total));
@@ -1183,16 +1208,77 @@ struct SystemImpl final : snh_system {
         return n;
     }
 
+    StateMap state_map() const { return {C.reps, d_rsite, R, total, G}; }
+
+    // Two chunks of device and pinned host memory for transfers of `need` bytes.
+    void ensure_transfer(size_t need)
+    {
+        const size_t want = std::min(std::max<size_t>(need, 4096), kChunkBytes);
+        if (xfer.bytes >= want) return;
+        xfer.release();
+        for (int k = 0; k < 2; k++) {
+            SNH_HIP(hipMalloc(&xfer.dev[k], want));
+            SNH_HIP(hipHostMalloc(&xfer.pin[k], want, hipHostMallocDefault));
+            SNH_HIP(hipEventCreateWithFlags(&xfer.ev[k], hipEventDisableTiming));
+        }
+        xfer.bytes = want;
+    }
+
+    // n items of `size` bytes to the host, chunk after chunk: pack(k0, m, dev)
+    // queues the items k0 .. k0 + m - 1 into device memory, put(k0, m, host)
+    // takes them from pinned memory while the next chunk is copied.
+    template <typename Pack, typename Put>
+    void stream_out(long long n, size_t size, Pack pack, Put put)
+    {
+        if (n <= 0) return;
+        ensure_transfer((size_t)n * size);
+        const long long per = (long long)(xfer.bytes / size), nch = (n + per - 1) / per;
+        auto issue = [&](long long c) {
+            const long long k0 = c * per, m = std::min(per, n - k0);
+            pack(k0, m, xfer.dev[c & 1]);
+            SNH_HIP(hipGetLastError());
+            SNH_HIP(hipMemcpyAsync(xfer.pin[c & 1], xfer.dev[c & 1], (size_t)m * size, hipMemcpyDeviceToHost, st));
+            SNH_HIP(hipEventRecord(xfer.ev[c & 1], st));
+        };
+        issue(0);
+        for (long long c = 0; c < nch; c++) {
+            if (c + 1 < nch) issue(c + 1);
+            SNH_HIP(hipEventSynchronize(xfer.ev[c & 1]));
+            const long long k0 = c * per;
+            put(k0, std::min(per, n - k0), xfer.pin[c & 1]);
+        }
+        check_resident();
+    }
+
     void download_planes(const T* P, int np, double* x)
     {
-        std::vector<T> h((size_t)np * total);
-        SNH_HIP(hipMemcpyAsync(h.data(), P, sizeof(T) * h.size(), hipMemcpyDeviceToHost, st));
+        const StateMap M = state_map();
+        stream_out(
+            interior_sites() * np, sizeof(T),
+            [&](long long k0, long long m, void* dev) { launch_state_pack<T>(M, P, np, k0, m, (T*)dev, st); },
+            [&](long long k0, long long m, const void* host) {
+                const T* h = static_cast<const T*>(host);
+                for (long long k = 0; k < m; k++) x[k0 + k] = (double)h[k];
+            });
+    }
+
+    void upload_planes(const double* x, int np, T* P)
+    {
+        const StateMap M = state_map();
+        const long long n = interior_sites();
+        ensure_transfer((size_t)n * np * sizeof(T));
+        const long long per = (long long)(xfer.bytes / (np * sizeof(T)));
+        for (long long s0 = 0, c = 0; s0 < n; s0 += per, c++) {
+            const long long m = std::min(per, n - s0);
+            SNH_HIP(hipEventSynchronize(xfer.ev[c & 1]));  // its last copy is done
+            T* h = static_cast<T*>(xfer.pin[c & 1]);
+            for (long long k = 0; k < m * np; k++) h[k] = (T)x[s0 * np + k];
+            SNH_HIP(hipMemcpyAsync(xfer.dev[c & 1], h, (size_t)m * np * sizeof(T), hipMemcpyHostToDevice, st));
+            SNH_HIP(hipEventRecord(xfer.ev[c & 1], st));
+            launch_state_unpack<T>(M, (const T*)xfer.dev[c & 1], np, s0, m, P, st);
+        }
+        SNH_HIP(hipGetLastError());
         SNH_HIP(hipStreamSynchronize(st));
-        check_resident();
-        for_each_padded([&](uint32_t g, long long s, bool interior) {
-            if (!interior) return;
-            for (int p = 0; p < np; p++) x[(size_t)np * s + p] = (double)h[(size_t)p * total + g];
-        });
     }
 
     int64_t total_sites() const override { return interior_sites(); }
@@ -1204,12 +1290,7 @@ struct SystemImpl final : snh_system {
         dz_valid = false;
         SNH_REQUIRE(coherent == (N > 0), SNH_ERR_INVALID,
                     coherent ? "coherent states require :SUN mode" : "in :SUN mode set coherent states");
-        std::vector<T> h((size_t)planes * total, (T)0);
-        for_each_padded([&](uint32_t g, long long s, bool) {
-            for (int p = 0; p < planes; p++) h[(size_t)p * total + g] = (T)x[(size_t)planes * s + p];
-        });
-        SNH_HIP(hipMemcpyAsync(X, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice, st));
-        SNH_HIP(hipStreamSynchronize(st));
+        upload_planes(x, planes, X);
     }
 
     void get_state(double* x, bool coherent) override
@@ -1218,10 +1299,16 @@ struct SystemImpl final : snh_system {
             SNH_REQUIRE(!coherent || N > 0, SNH_ERR_INVALID, "coherent states require :SUN mode");
             download_planes(X, planes, x);
         } else {
-            // dipoles of a coherent state: expected_spin(Z) (Integrators.jl:354)
-            launch_sun_expected_spin<T>(C, nblocks, X, Xp, st);  // stage buffer is free between steps
-            SNH_HIP(hipGetLastError());
-            download_planes(Xp, 3, x);
+            // dipoles of a coherent state: expected_spin(Z) (Integrators.jl:354), in FP64
+            const StateMap M = state_map();
+            stream_out(
+                interior_sites(), 3 * sizeof(double),
+                [&](long long k0, long long m, void* dev) {
+                    launch_state_spin<T>(M, X, N, k0, m, (double*)dev, st);
+                },
+                [&](long long k0, long long m, const void* host) {
+                    std::memcpy(x + 3 * k0, host, (size_t)m * 3 * sizeof(double));
+                });
         }
     }
 
@@ -1485,21 +1572,17 @@ struct SystemImpl final : snh_system {
         SNH_REQUIRE(corr.nt > 0, SNH_ERR_INVALID, "sampled correlations are not initialised");
         const int nt = corr.nt, nc = corr.ncorr;
         const long long ncell = corr.ncell;
-        const size_t n = (size_t)nc * na * nt * na * ncell;
-        std::vector<double> h(2 * n);
-        SNH_HIP(hipMemcpyAsync(h.data(), corr.data, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st));
-        SNH_HIP(hipStreamSynchronize(st));
         if (out)
-            for (int c = 0; c < nc; c++)
-                for (int i = 0; i < na; i++)
-                    for (int k = 0; k < nt; k++)
-                        for (int j = 0; j < na; j++)
-                            for (long long q = 0; q < ncell; q++) {
-                                const size_t src = ((((size_t)c * na + i) * nt + k) * na + j) * ncell + q;
-                                const size_t dst = c + (size_t)nc * (i + (size_t)na * (j + (size_t)na * (q + ncell * k)));
-                                out[2 * dst] = h[2 * src];
-                                out[2 * dst + 1] = h[2 * src + 1];
-                            }
+            stream_out(
+                (long long)nc * na * nt * na * ncell, 2 * sizeof(double),
+                [&](long long k0, long long m, void* dev) {
+                    launch_corr_pack(corr.data, nc, na, nt, ncell, k0, m, dev, st);
+                },
+                [&](long long k0, long long m, const void* host) {
+                    std::memcpy(out + 2 * k0, host, (size_t)m * 2 * sizeof(double));
+                });
+        else
+            SNH_HIP(hipStreamSynchronize(st));
         if (nsamples) *nsamples = corr.nsamples;
     }
 
@@ -2309,16 +2392,7 @@ struct SystemImpl final : snh_system {
             }
             SNH_HIP(hipMemcpyAsync(Xsave, X, bytes, hipMemcpyDeviceToDevice, st));
             SNH_HIP(hipMemsetAsync(dgrad, 0, sizeof(double) * std::max(1, nparams), st));
-            SNH_HIP(hipMemsetAsync(lam, 0, bytes, st));
-            {
-                std::vector<T> h(np, (T)0);
-                for_each_padded([&](uint32_t gi, long long si, bool interior) {
-                    if (!interior) return;
-                    for (int a = 0; a < 3; a++) h[(size_t)a * total + gi] = (T)dLdS[3 * (size_t)si + a];
-                });
-                SNH_HIP(hipMemcpyAsync(lam, h.data(), bytes, hipMemcpyHostToDevice, st));
-                SNH_HIP(hipStreamSynchronize(st));
-            }
+            upload_planes(dLdS, 3, lam);
             const T tdt = (T)rec_dt;
             const int ncp = (int)ckpt.size();
             for (int seg = ncp - 1; seg >= 0; seg--) {

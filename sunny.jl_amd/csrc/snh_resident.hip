@@ -157,7 +157,7 @@ __device__ __forceinline__ Part<T> res_part(const Couplings<T>& C, const ResArgs
 // are those of local_field.  An isotropic bond is one fused multiply-add per
 // component in the launched Heun stages and a product and a sum in the
 // launched midpoint sweeps (whose general form the compiler cannot fuse);
-// kFused follows suit, so that states agree bitwise.
+// kFused follows suit, so that FP64 states agree bitwise.
 template <typename T, int CH, bool kIso, bool kFused>
 __device__ __forceinline__ V3<T> res_field(const Couplings<T>& C, const Part<T>& P, const T* b, V3<T> s)
 {

@@ -22,17 +22,12 @@ __device__ __forceinline__ V3<T> cross3(V3<T> a, V3<T> b)
     return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
 
-// |s|^2 with its two fused multiply-adds spelled out: which product of a sum
-// of squares the compiler would fuse differs from kernel to kernel, and the
-// launched and the resident steps agree bitwise.
+// |s|^2 in FP64 with its two fused multiply-adds spelled out: which product of
+// a sum of squares the compiler would fuse differs from kernel to kernel, and
+// the launched and the resident FP64 steps agree bitwise.
 __device__ __forceinline__ double norm2(V3<double> s)
 {
     return __builtin_fma(s.z, s.z, __builtin_fma(s.y, s.y, s.x * s.x));
-}
-
-__device__ __forceinline__ float norm2(V3<float> s)
-{
-    return __builtin_fmaf(s.z, s.z, __builtin_fmaf(s.y, s.y, s.x * s.x));
 }
 
 // kappa * s/|s| (normalize_dipole, System.jl:421-423).  FP64 state:
@@ -49,7 +44,7 @@ __device__ __forceinline__ V3<double> normalize_dipole(V3<double> s, double kapp
 __device__ __forceinline__ V3<float> normalize_dipole(V3<float> s, float kappa)
 {
     if (kappa == 0.0f) return {0, 0, 0};
-    const float f = kappa * __builtin_amdgcn_rsqf(norm2(s));
+    const float f = kappa * __builtin_amdgcn_rsqf(s.x * s.x + s.y * s.y + s.z * s.z);
     return {s.x * f, s.y * f, s.z * f};
 }
 
@@ -74,7 +69,7 @@ __device__ __forceinline__ V3<float> normalize_dipole_mu(V3<float> s, float kapp
         mu = 0;
         return {0, 0, 0};
     }
-    const float f = kappa * __builtin_amdgcn_rsqf(norm2(s));
+    const float f = kappa * __builtin_amdgcn_rsqf(s.x * s.x + s.y * s.y + s.z * s.z);
     mu = __builtin_amdgcn_rcpf(f);
     return {s.x * f, s.y * f, s.z * f};
 }

@@ -95,9 +95,8 @@ class SampledCorrelations:
         """sc.data as complex [ncorr, na, na, L1, L2, L3, n_all_omega]."""
         nc, na = len(self.corr_pairs), self.na
         L1, L2, L3 = self.dims
-        buf = np.zeros(2 * nc * na * na * L1 * L2 * L3 * self.n_all_omega)
-        self.sys._device().call("snh_corr_data", _lib.dptr(buf), None)
-        z = buf[0::2] + 1j * buf[1::2]
+        z = np.empty(nc * na * na * L1 * L2 * L3 * self.n_all_omega, complex)
+        self.sys._device().call("snh_corr_data", _lib.dptr(z.view(float)), None)
         # column-major (Julia) order: reverse the axes of a C-order view
         return z.reshape(self.n_all_omega, L3, L2, L1, na, na, nc).transpose(6, 5, 4, 3, 2, 1, 0)
 

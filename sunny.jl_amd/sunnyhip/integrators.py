@@ -160,6 +160,7 @@ class ReplicaBatch:
         self._handle = None
         self._host_dirty = True
         self._dev_dirty = False
+        self._dip = self._coh = None
         self.nsites = sum(s.nsites for s in self.systems)
 
     def _device(self):
@@ -171,8 +172,7 @@ class ReplicaBatch:
                 self._handle.call("snh_set_dipoles", _lib.dptr(np.ascontiguousarray(x)))
             else:
                 z = np.concatenate([s.coherents_flat() for s in self.systems])
-                x = np.ascontiguousarray(np.stack([z.real, z.imag], -1))
-                self._handle.call("snh_set_coherents", _lib.dptr(x))
+                self._handle.call("snh_set_coherents", _lib.dptr(z.view(float)))
             self._host_dirty = False
         return self._handle
 
@@ -181,20 +181,16 @@ class ReplicaBatch:
         if not self._dev_dirty:
             return
         h = self._handle
-        d = np.empty((h.total, 3))
-        h.call("snh_get_dipoles", _lib.dptr(d))
-        z = None
-        if self.N > 0:
-            zz = np.empty((h.total, self.N, 2))
-            h.call("snh_get_coherents", _lib.dptr(zz))
-            z = zz[..., 0] + 1j * zz[..., 1]
+        if self._dip is None:  # where the device's states land, kept between calls
+            self._dip = np.empty((h.total, 3))
+            self._coh = np.empty((h.total, self.N), complex) if self.N > 0 else None
+        h.call("snh_get_dipoles", _lib.dptr(self._dip))
+        if self.N > 0:  # complex entries are the ABI's (re, im) pairs
+            h.call("snh_get_coherents", _lib.dptr(self._coh.view(float)))
         o = 0
         for s in self.systems:
             n = s.nsites
-            if self.N == 0:
-                s.set_state_flat(dip=d[o:o + n])
-            else:
-                s.set_state_flat(coh=z[o:o + n])
+            s._replace_state(self._dip[o:o + n], self._coh[o:o + n] if self.N > 0 else None)
             o += n
         self._dev_dirty = False
 

@@ -109,13 +109,9 @@ class System:
     def _pull(self):
         if self._dev_dirty:
             h = self._handle
-            d = np.empty((h.total, 3))
-            h.call("snh_get_dipoles", _lib.dptr(d))
-            self._dip[:] = d
-            if self.N > 0:
-                z = np.empty((h.total, self.N, 2))
-                h.call("snh_get_coherents", _lib.dptr(z))
-                self._coh[:] = z[..., 0] + 1j * z[..., 1]
+            h.call("snh_get_dipoles", _lib.dptr(self._dip))
+            if self.N > 0:  # complex entries are the ABI's (re, im) pairs
+                h.call("snh_get_coherents", _lib.dptr(self._coh.view(float)))
             self._dev_dirty = False
 
     @property
@@ -147,6 +143,14 @@ class System:
             self._dip[:] = expected_spin_host(self._coh, self.N)
         elif dip is not None:
             self._dip[:] = np.asarray(dip).reshape(self.nsites, 3)
+        self._host_dirty = True
+
+    def _replace_state(self, dip, coh):
+        """The whole state, dipoles being the expected spins of the kets."""
+        self._dip[:] = dip
+        if coh is not None:
+            self._coh[:] = coh
+        self._dev_dirty = False
         self._host_dirty = True
 
     def site_kappas(self):
@@ -237,8 +241,8 @@ class System:
             if self.N == 0:
                 h.call("snh_set_dipoles", _lib.dptr(np.ascontiguousarray(self._dip)))
             else:
-                z = np.ascontiguousarray(np.stack([self._coh.real, self._coh.imag], -1))
-                h.call("snh_set_coherents", _lib.dptr(z))
+                z = np.ascontiguousarray(self._coh)
+                h.call("snh_set_coherents", _lib.dptr(z.view(float)))
             self._host_dirty = False
         return self._handle
 
