@@ -105,7 +105,8 @@ std::vector<double> quadrupole_ops(int N)
 // candidates that fit the LDS.  Cost of one workgroup = (layers loaded) x
 // (positions per layer) + 3 x (site lanes computed, idle lanes included),
 // each divided by the fraction of a 128-byte line its rows fill; a CU works
-// through ceil(workgroups / CUs) of them, 1.3x slower when only one fits.
+// through ceil(workgroups / CUs) of them, 1.3x slower when only one fits or
+// only one is there.
 struct TilePlan {
     TileArgs A{};
     int threads = 0;
@@ -202,7 +203,7 @@ bool plan_tiles(int na, const int w[3], const std::vector<std::array<int, 3>>& d
                 // rows shorter than a 128-byte line waste load and store bandwidth
                 const double eff_ld = std::min(1.0, (double)ROW * elem / 128.0);
                 const double eff_st = std::min(1.0, (double)T1 * elem / 128.0);
-                const double bubble = per_cu >= 2 ? 1.0 : 1.3;
+                const double bubble = per_cu >= 2 && rounds >= 2 ? 1.0 : 1.3;
                 const double cost = (double)rounds * bubble *
                                     ((double)(kseg + 2 * w[2]) * npos / eff_ld + 3.0 * kseg * nsite / eff_st);
                 {
@@ -678,6 +679,7 @@ struct SystemImpl final : snh_system {
                     "layout must be SNH_LAYOUT_AUTO or SNH_LAYOUT_GHOST");
         // one small :dipole replica without Ewald, above the one-workgroup
         // size: steps in one cooperative launch
+        int ncu = 1;
         const long long sites1 = sp.nreplicas == 1 ? (long long)sp.dims[0] * sp.dims[1] * sp.dims[2] * na : 0;
         coop = N == 0 && !ewald && R == 1 && sites1 > kResOneWg &&
                sites1 <= std::min(env_int("SNH_COOP_MAX_SITES", kResMaxSites), kResMaxSites) &&
@@ -698,6 +700,7 @@ struct SystemImpl final : snh_system {
             tiled = plan_tiles(na, w, dv, sizeof(T), prop.sharedMemPerBlock - 256, lds_cu,
                                std::max(1, prop.multiProcessorCount), tile_cands, 16);
             if (tiled) tp = tile_cands[0];
+            ncu = std::max(1, prop.multiProcessorCount);
         }
         // the tiled sweep fetches halos with the periodic wrap itself: no ghosts
         const int lw[3] = {tiled ? 0 : w[0], tiled ? 0 : w[1], tiled ? 0 : w[2]};
@@ -942,8 +945,9 @@ struct SystemImpl final : snh_system {
         if (tiled) {
             // lean FP32 kernels over isotropic bonds run both stages one site
             // per thread on the model's first tile where it offers that plan
-            apply_plan(tile_cands[default_correct_plan()], 0);
-            apply_plan(tile_cands[default_correct_plan()], 1);
+            const size_t dp = default_correct_plan(ncu);
+            apply_plan(tile_cands[dp], 0);
+            apply_plan(tile_cands[dp], 1);
         }
         if (!partial) {
             partial_cap = std::max<size_t>(nblocks, 1);
@@ -1334,18 +1338,30 @@ struct SystemImpl final : snh_system {
     // The plan of both stages (and of the midpoint iteration) before any
     // autotuning: the cost model's first, except that lean FP32 kernels over
     // isotropic bonds take the same tile with one site per thread where the
-    // model offers it (their one-site forms fit two 1024-thread workgroups
-    // per CU: the corrector in 64 registers, the predictor in 60).
-    size_t default_correct_plan() const
+    // model offers it: their one-site forms fit two 1024-thread workgroups
+    // per CU (the corrector in 64 registers, the predictor in 60), so axis 3
+    // is cut where a CU then has two at least, by the same count of layers
+    // loaded (1.3 for a lone workgroup).  8 pyrochlore replicas of 32^3 x 16:
+    // 95.5 us per step with 256 workgroups, 84.5 with 512.
+    size_t default_correct_plan(int ncu) const
     {
         if (sizeof(T) != 4 || !C.lean_ok || !C.iso || ewald || env_int("SNH_TILE_SP", 0)) return 0;
         const TilePlan& b = tile_cands[0];
-        for (size_t k = 1; k < tile_cands.size(); k++) {
+        size_t best = 0;
+        double least = 0;
+        for (size_t k = 0; k < tile_cands.size(); k++) {
             const TilePlan& a = tile_cands[k];
-            if (a.A.sp == 1 && b.A.sp == 2 && a.A.T1 == b.A.T1 && a.A.T2 == b.A.T2 && a.work.size() == b.work.size())
-                return k;
+            if (a.A.sp != 1 || a.A.T1 != b.A.T1 || a.A.T2 != b.A.T2) continue;
+            int layers = 0;
+            for (const TileWork& w : a.work) layers = std::max(layers, w.k1 - w.k0);
+            const int rounds = ((int)a.work.size() + ncu - 1) / ncu;
+            const double cost = rounds * (layers + 2 * a.A.w3) * (rounds == 1 ? 1.3 : 1.0);
+            if (least == 0 || cost < least) {
+                least = cost;
+                best = k;
+            }
         }
-        return 0;
+        return best;
     }
 
     void apply_plan(const TilePlan& P, int which)
