@@ -74,7 +74,8 @@ __global__ __launch_bounds__(kCorrThreads) void k_corr_lines(Cd* __restrict__ bu
         base = l;
         stride = L1 * L2;
     }
-    line_c2c<double>(buf + f * ncell, (int)base, stride, L, tw);
+    // this thread's line only
+    lines_c2c<kLmax, 1>(buf + f * ncell, (int)threadIdx.x + 1, [&](int) { return base; }, stride, L, tw);
 }
 
 // Direct DFT over the T time slots of nl independent lines ([T][nl] layout):

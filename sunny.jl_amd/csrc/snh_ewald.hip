@@ -38,6 +38,7 @@
 
 #include <hipfft/hipfft.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <map>
 #include <mutex>
@@ -46,6 +47,10 @@ namespace snh {
 
 constexpr int kFftThreads = 256;
 constexpr int kSpecKB = 16;  // wavevectors per spectrum block (128-byte runs in FP32)
+// The transforms take three fields a workgroup up to this LDS (two workgroups
+// per CU) and from this count of workgroups (sublattices x replicas).
+constexpr size_t kFieldsLds3 = 80 * 1024;
+constexpr int kFieldsMin3 = 256;
 
 // ---------------------------------------------------------------------------
 // One workgroup transforms one field.  Dynamic LDS: spectrum [nk] complex,
@@ -81,33 +86,65 @@ __device__ __forceinline__ FftLds<T> fft_lds(const EwaldGeom& G)
 template <typename T>
 __device__ __forceinline__ void fwd3d(const EwaldGeom& G, const FftLds<T>& F)
 {
-    for (int line = threadIdx.x; line < G.L2 * G.L3; line += blockDim.x)
-        line_r2c<T>(F.fld + line * F.row, F.spec + G.H1 * line, G.L1, F.tw1);
+    lines_r2c<kLmax, T>(
+        G.L2 * G.L3, [&](int l) { return F.fld + l * F.row; }, [&](int l) { return F.spec + G.H1 * l; }, G.L1, F.tw1);
     __syncthreads();
-    for (int line = threadIdx.x; line < G.H1 * G.L3; line += blockDim.x) {
-        const int k1 = line % G.H1, c3 = line / G.H1;
-        line_c2c<T>(F.spec, k1 + G.H1 * G.L2 * c3, G.H1, G.L2, F.tw2);
-    }
+    lines_c2c<kLmax, -1>(
+        F.spec, G.H1 * G.L3, [&](int l) { return l % G.H1 + G.H1 * G.L2 * (l / G.H1); }, G.H1, G.L2, F.tw2);
     __syncthreads();
-    for (int line = threadIdx.x; line < G.H1 * G.L2; line += blockDim.x)
-        line_c2c<T>(F.spec, line, G.H1 * G.L2, G.L3, F.tw3);
+    lines_c2c<kLmax, -1>(F.spec, G.H1 * G.L2, [&](int l) { return l; }, G.H1 * G.L2, G.L3, F.tw3);
     __syncthreads();
 }
 
-// Backward c2r 3D FFT of F.spec into F.fld (unscaled).  Twiddles sign +1.
+// NF fields of one workgroup transformed in place: dynamic LDS holds their
+// half spectra [NF][nk] complex and three twiddle tables [kLmax]; a real line
+// lies in the storage of its own half spectrum (H1 complex values, of which
+// L1 words are the line).
 template <typename T>
-__device__ __forceinline__ void inv3d(const EwaldGeom& G, const FftLds<T>& F)
-{
-    for (int line = threadIdx.x; line < G.H1 * G.L2; line += blockDim.x)
-        line_c2c<T>(F.spec, line, G.H1 * G.L2, G.L3, F.tw3);
-    __syncthreads();
-    for (int line = threadIdx.x; line < G.H1 * G.L3; line += blockDim.x) {
-        const int k1 = line % G.H1, c3 = line / G.H1;
-        line_c2c<T>(F.spec, k1 + G.H1 * G.L2 * c3, G.H1, G.L2, F.tw2);
+struct FieldsLds {
+    C2<T>* spec;
+    C2<T>* tw1;
+    C2<T>* tw2;
+    C2<T>* tw3;
+    __device__ __forceinline__ T* line(const EwaldGeom& G, int l) const
+    {
+        return reinterpret_cast<T*>(spec + G.H1 * l);
     }
+};
+
+template <typename T, int NF>
+__device__ __forceinline__ FieldsLds<T> fields_lds(const EwaldGeom& G)
+{
+    extern __shared__ __align__(16) unsigned char snh_lds[];
+    FieldsLds<T> F;
+    F.spec = reinterpret_cast<C2<T>*>(snh_lds);
+    F.tw1 = F.spec + NF * G.nk;
+    F.tw2 = F.tw1 + kLmax;
+    F.tw3 = F.tw2 + kLmax;
+    return F;
+}
+
+size_t ewald_fields_lds_bytes(const EwaldGeom& G, int nf, size_t elem)
+{
+    return ((size_t)nf * G.nk + 3 * kLmax) * 2 * elem;
+}
+
+// In-place forward (S = -1) and backward (S = +1) c2c transforms of NF half
+// spectra along axis 2 or 3.
+template <int kMax, int S, typename T>
+__device__ __forceinline__ void fields_axis2(const EwaldGeom& G, const FieldsLds<T>& F, int nf)
+{
+    lines_c2c<kMax, S>(
+        F.spec, nf * G.H1 * G.L3, [&](int l) { return l % G.H1 + G.H1 * G.L2 * (l / G.H1); }, G.H1, G.L2, F.tw2);
     __syncthreads();
-    for (int line = threadIdx.x; line < G.L2 * G.L3; line += blockDim.x)
-        line_c2r<T>(F.spec + G.H1 * line, F.fld + line * F.row, G.L1, F.tw1);
+}
+
+template <int kMax, int S, typename T>
+__device__ __forceinline__ void fields_axis3(const EwaldGeom& G, const FieldsLds<T>& F, int nf)
+{
+    const int p = G.H1 * G.L2;
+    lines_c2c<kMax, S>(
+        F.spec, nf * p, [&](int l) { return l % p + p * G.L3 * (l / p); }, p, G.L3, F.tw3);
     __syncthreads();
 }
 
@@ -124,31 +161,47 @@ __device__ __forceinline__ uint32_t ewald_site(const EwaldGeom& G, uint32_t off,
     return off + (uint32_t)((c1 + G.w1) + G.P1 * ((c2 + G.w2) + G.P2 * (c3 + G.w3))) + G.pcell * (uint32_t)j;
 }
 
-// Forward transform of mu = -g S.  grid = (3 na, R); field f = 3 j + beta.
-template <typename T>
-__global__ __launch_bounds__(kFftThreads) void k_ewald_fwd(EwaldGeom G, int R, const ReplicaInfo* __restrict__ reps,
-                                                           uint32_t total, const T* __restrict__ gmat,
-                                                           const T* __restrict__ S, C2<T>* __restrict__ Fmu)
+// Forward transform of mu = -g S.  A workgroup transforms NF fields of one
+// replica: NF = 3, the three components of a sublattice (grid (na, R)), or
+// NF = 1 (grid (3 na, R)).  Three together read the sublattice's spins once
+// and write 384-byte runs of the spectra; in place they take 55 KB of LDS on
+// a 16^3 FP32 grid, two workgroups of 768 threads per CU.  One field a
+// workgroup has the three components on different XCDs, each reading the
+// spins from beyond its L2, and had half its LDS in a real copy: the field of
+// the 16^3 x 16 pyrochlore 93.6 -> 74.6 us at 32 replicas, 57.3 -> 49.1 at 16,
+// but 45.7 -> 47.8 at 8, whose 128 workgroups leave half the chip idle (one
+// field a workgroup, in place: 43.2).
+template <typename T, int NF, int kMax>
+__global__ __attribute__((amdgpu_waves_per_eu(NF == 3 ? 6 : 1)))
+__launch_bounds__(NF * kFftThreads) void k_ewald_fwd(EwaldGeom G, int R,
+                                                                const ReplicaInfo* __restrict__ reps, uint32_t total,
+                                                                const T* __restrict__ gmat, const T* __restrict__ S,
+                                                                C2<T>* __restrict__ Fmu)
 {
-    const int f = blockIdx.x, r = blockIdx.y;
-    const int j = f / 3, beta = f % 3;
-    const FftLds<T> F = fft_lds<T>(G);
+    constexpr int NT = NF * kFftThreads;
+    const int f0 = NF * (int)blockIdx.x, r = blockIdx.y;  // first field
+    const int j = f0 / 3;
+    const FieldsLds<T> F = fields_lds<T, NF>(G);
     const uint32_t off = reps[r].off;
-    const T g0 = gmat[9 * j + 3 * beta], g1 = gmat[9 * j + 3 * beta + 1], g2 = gmat[9 * j + 3 * beta + 2];
+    T gm[NF][3];
+#pragma unroll
+    for (int q = 0; q < NF; q++)
+#pragma unroll
+        for (int a = 0; a < 3; a++) gm[q][a] = gmat[3 * (f0 + q) + a];
     // loads in flight per thread: a 16^3 grid in one round
-    constexpr int kBatch = sizeof(T) == 4 ? 16 : 8;
-    for (int c0 = 0; c0 < G.ncell; c0 += kBatch * kFftThreads) {
-        T v[kBatch];
+    constexpr int kBatch = NF == 3 ? 6 : sizeof(T) == 4 ? 16 : 8;
+    for (int c0 = 0; c0 < G.ncell; c0 += kBatch * NT) {
+        T v[kBatch][3];
         // unconditional loads (a cell past the end reads cell 0 and is
         // dropped), so that all of them are in flight before the first wait
 #pragma unroll
         for (int q = 0; q < kBatch; q++) {
-            const int c = c0 + q * kFftThreads + threadIdx.x;
+            const int c = c0 + q * NT + threadIdx.x;
             const int cc = c < G.ncell ? c : 0;
             const int c1 = cc % G.L1, l = cc / G.L1;
             const uint32_t g = ewald_site(G, off, j, c1, l % G.L2, l / G.L2);
-            const T m = -(g0 * ldg(S, g) + g1 * ldg(S + total, g) + g2 * ldg(S + 2 * (size_t)total, g));
-            v[q] = c < G.ncell ? m : (T)0;
+#pragma unroll
+            for (int a = 0; a < 3; a++) v[q][a] = ldg(S + a * (size_t)total, g);
         }
         if (c0 == 0) {  // while the first loads are in flight
             make_twiddles(F.tw1, G.L1, -1);
@@ -157,13 +210,25 @@ __global__ __launch_bounds__(kFftThreads) void k_ewald_fwd(EwaldGeom G, int R, c
         }
 #pragma unroll
         for (int q = 0; q < kBatch; q++) {
-            const int c = c0 + q * kFftThreads + threadIdx.x;
-            if (c < G.ncell) F.fld[(c / G.L1) * F.row + c % G.L1] = v[q];
+            const int c = c0 + q * NT + threadIdx.x;
+            if (c >= G.ncell) continue;
+            const int c1 = c % G.L1, l = c / G.L1;
+#pragma unroll
+            for (int b = 0; b < NF; b++)
+                F.line(G, l + b * G.L2 * G.L3)[c1] = -(gm[b][0] * v[q][0] + gm[b][1] * v[q][1] + gm[b][2] * v[q][2]);
         }
     }
     __syncthreads();
-    fwd3d<T>(G, F);
-    for (int k = threadIdx.x; k < G.nk; k += blockDim.x) Fmu[spec_index(G, R, r, f, k)] = F.spec[k];
+    lines_r2c<kMax, T>(
+        NF * G.L2 * G.L3, [&](int l) { return F.line(G, l); }, [&](int l) { return F.spec + G.H1 * l; }, G.L1, F.tw1);
+    __syncthreads();
+    fields_axis2<kMax, -1>(G, F, NF);
+    fields_axis3<kMax, -1>(G, F, NF);
+    for (int t = threadIdx.x;; t += NT) {  // blocks of kSpecKB wavevectors, field after field
+        const int k = t / (NF * kSpecKB) * kSpecKB + t % kSpecKB, q = t / kSpecKB % NF;
+        if (t >= (int)(G.nk + kSpecKB - 1) / kSpecKB * kSpecKB * NF) break;
+        if (k < G.nk) Fmu[spec_index(G, R, r, f0 + q, k)] = F.spec[q * G.nk + k];
+    }
 }
 
 // Forward transform of the real-space tensor A (FP64), written as the
@@ -331,46 +396,55 @@ __global__ __launch_bounds__(256 * NRT) void k_ewald_contract_mfma(EwaldGeom G, 
 }
 
 // Inverse: c2r 3D FFT of F[phi] scaled by 1/Ncell -> phi plane alpha of
-// sublattice i (stored as O: T, or FP64 for the Metropolis potential).
-// grid = (3 na, R); field = 3 i + alpha.
-template <typename T, typename O>
-__global__ __launch_bounds__(kFftThreads) void k_ewald_inv(EwaldGeom G, int R, const ReplicaInfo* __restrict__ reps,
-                                                           uint32_t total, const C2<T>* __restrict__ Fphi,
-                                                           O* __restrict__ phi)
+// sublattice i (stored as O: T, or FP64 for the Metropolis potential), NF
+// fields 3 i + alpha a workgroup as in the forward transform.
+template <typename T, typename O, int NF, int kMax>
+__global__ __attribute__((amdgpu_waves_per_eu(NF == 3 ? 6 : 1)))
+__launch_bounds__(NF * kFftThreads) void k_ewald_inv(EwaldGeom G, int R,
+                                                                const ReplicaInfo* __restrict__ reps, uint32_t total,
+                                                                const C2<T>* __restrict__ Fphi, O* __restrict__ phi)
 {
-    const int f = blockIdx.x, r = blockIdx.y;
-    const int i = f / 3, alpha = f % 3;
-    const FftLds<T> F = fft_lds<T>(G);
+    constexpr int NT = NF * kFftThreads;
+    const int f0 = NF * (int)blockIdx.x, r = blockIdx.y;
+    const FieldsLds<T> F = fields_lds<T, NF>(G);
+    const int nt = (int)(G.nk + kSpecKB - 1) / kSpecKB * kSpecKB * NF;
     // loads in flight per thread: the half spectrum of a 16^3 grid in one round
-    constexpr int kBatch = sizeof(T) == 4 ? 12 : 6;
-    for (int k0 = 0; k0 < G.nk; k0 += kBatch * kFftThreads) {
+    constexpr int kBatch = NF == 3 ? 9 : sizeof(T) == 4 ? 12 : 6;
+    for (int t0 = 0; t0 < nt; t0 += kBatch * NT) {
         C2<T> v[kBatch];
         // unconditional loads (past the end: wavevector 0, dropped below)
 #pragma unroll
-        for (int q = 0; q < kBatch; q++) {
-            const int k = k0 + q * kFftThreads + threadIdx.x;
-            v[q] = Fphi[spec_index(G, R, r, f, k < G.nk ? k : 0)];
+        for (int b = 0; b < kBatch; b++) {
+            const int t = t0 + b * NT + threadIdx.x;
+            const int k = t / (NF * kSpecKB) * kSpecKB + t % kSpecKB, q = t / kSpecKB % NF;
+            v[b] = Fphi[spec_index(G, R, r, f0 + q, k < G.nk ? k : 0)];
         }
-        if (k0 == 0) {  // while the first loads are in flight
+        if (t0 == 0) {  // while the first loads are in flight
             make_twiddles(F.tw1, G.L1, +1);
             make_twiddles(F.tw2, G.L2, +1);
             make_twiddles(F.tw3, G.L3, +1);
         }
 #pragma unroll
-        for (int q = 0; q < kBatch; q++) {
-            const int k = k0 + q * kFftThreads + threadIdx.x;
-            if (k < G.nk) F.spec[k] = v[q];
+        for (int b = 0; b < kBatch; b++) {
+            const int t = t0 + b * NT + threadIdx.x;
+            const int k = t / (NF * kSpecKB) * kSpecKB + t % kSpecKB, q = t / kSpecKB % NF;
+            if (k < G.nk) F.spec[q * G.nk + k] = v[b];
         }
     }
     __syncthreads();
-    inv3d<T>(G, F);
+    fields_axis3<kMax, 1>(G, F, NF);
+    fields_axis2<kMax, 1>(G, F, NF);
+    lines_c2r<kMax, T>(
+        NF * G.L2 * G.L3, [&](int l) { return F.spec + G.H1 * l; }, [&](int l) { return F.line(G, l); }, G.L1, F.tw1);
+    __syncthreads();
     const T scale = (T)(1.0 / (double)G.ncell);
-    O* const out = phi + (size_t)alpha * total;
     const uint32_t off = reps[r].off;
-    for (int c = threadIdx.x; c < G.ncell; c += blockDim.x) {
+    for (int t = threadIdx.x; t < NF * G.ncell; t += NT) {
+        const int q = t / (int)G.ncell, c = t % (int)G.ncell;
         const int c1 = c % G.L1, l = c / G.L1;
-        const T v = F.fld[l * F.row + c1] * scale;
-        stg(out, ewald_site(G, off, i, c1, l % G.L2, l / G.L2), (O)v);
+        const int i = (f0 + q) / 3, alpha = (f0 + q) % 3;
+        const T v = F.line(G, l + q * G.L2 * G.L3)[c1] * scale;
+        stg(phi + (size_t)alpha * total, ewald_site(G, off, i, c1, l % G.L2, l / G.L2), (O)v);
     }
 }
 
@@ -476,15 +550,12 @@ __global__ __launch_bounds__(kFftThreads) void k_ewald_fwd_slab(EwaldGeom G, int
         }
     }
     __syncthreads();
-    for (int line = threadIdx.x; line < 3 * G.L2; line += blockDim.x) {
-        const int beta = line / G.L2, c2 = line % G.L2;
-        line_r2c<T>(F.fld + beta * F.plane + c2 * F.row, F.spec + beta * F.nkp + G.H1 * c2, G.L1, F.tw1);
-    }
+    // the three planes and their half spectra follow each other row by row
+    lines_r2c<kLmax, T>(
+        3 * G.L2, [&](int l) { return F.fld + l * F.row; }, [&](int l) { return F.spec + G.H1 * l; }, G.L1, F.tw1);
     __syncthreads();
-    for (int line = threadIdx.x; line < 3 * G.H1; line += blockDim.x) {
-        const int beta = line / G.H1, k1 = line % G.H1;
-        line_c2c<T>(F.spec + beta * F.nkp, k1, G.H1, G.L2, F.tw2);
-    }
+    lines_c2c<kLmax, -1>(
+        F.spec, 3 * G.H1, [&](int l) { return l % G.H1 + F.nkp * (l / G.H1); }, G.H1, G.L2, F.tw2);
     __syncthreads();
     for (int t = threadIdx.x; t < 3 * F.nkp; t += blockDim.x) {
         const int beta = t / F.nkp, k12 = t % F.nkp;
@@ -568,15 +639,11 @@ __global__ __launch_bounds__(kFftThreads) void k_ewald_inv_slab(EwaldGeom G, con
         F.spec[t] = {ar, ai};
     }
     __syncthreads();
-    for (int line = threadIdx.x; line < 3 * G.H1; line += blockDim.x) {
-        const int alpha = line / G.H1, k1 = line % G.H1;
-        line_c2c<T>(F.spec + alpha * F.nkp, k1, G.H1, G.L2, F.tw2);
-    }
+    lines_c2c<kLmax, 1>(
+        F.spec, 3 * G.H1, [&](int l) { return l % G.H1 + F.nkp * (l / G.H1); }, G.H1, G.L2, F.tw2);
     __syncthreads();
-    for (int line = threadIdx.x; line < 3 * G.L2; line += blockDim.x) {
-        const int alpha = line / G.L2, c2 = line % G.L2;
-        line_c2r<T>(F.spec + alpha * F.nkp + G.H1 * c2, F.fld + alpha * F.plane + c2 * F.row, G.L1, F.tw1);
-    }
+    lines_c2r<kLmax, T>(
+        3 * G.L2, [&](int l) { return F.spec + G.H1 * l; }, [&](int l) { return F.fld + l * F.row; }, G.L1, F.tw1);
     __syncthreads();
     const T scale = (T)(1.0 / (double)G.ncell);
     const uint32_t off = reps[r].off;
@@ -969,21 +1036,44 @@ bool launch_ewald_field(const EwaldGeom& G, int R, const ReplicaInfo* reps, uint
         }
         return true;
     }
-    const size_t lds = ewald_fft_lds_bytes(G, sizeof(T));
-    allow_dynamic_lds(reinterpret_cast<const void*>(&k_ewald_fwd<T>), lds);
-    hipLaunchKernelGGL(k_ewald_fwd<T>, dim3(3 * G.na, R), dim3(kFftThreads), lds, st, G, R, reps, total, gmat, S,
-                       reinterpret_cast<C2<T>*>(Fmu));
+    // three fields a workgroup (FP32) where two such workgroups fit a CU's
+    // LDS and there are workgroups for most CUs
+    const bool lines16 = std::max({G.L1, G.L2, G.L3}) <= kLineShort;
+    const bool three = sizeof(T) == 4 && lines16 && G.na * R >= kFieldsMin3 &&
+                       ewald_fields_lds_bytes(G, 3, sizeof(T)) <= kFieldsLds3;
+    const size_t lds = ewald_fields_lds_bytes(G, three ? 3 : 1, sizeof(T));
+    const dim3 grid((unsigned)(three ? G.na : 3 * G.na), (unsigned)R);
+    auto fwd = [&](auto nf, auto lmax) {
+        constexpr int NF = decltype(nf)::value, kMax = decltype(lmax)::value;
+        allow_dynamic_lds(reinterpret_cast<const void*>(&k_ewald_fwd<T, NF, kMax>), lds);
+        hipLaunchKernelGGL((k_ewald_fwd<T, NF, kMax>), grid, dim3(NF * kFftThreads), lds, st, G, R, reps, total, gmat,
+                           S, reinterpret_cast<C2<T>*>(Fmu));
+    };
+    auto inv = [&](auto nf, auto lmax) {
+        constexpr int NF = decltype(nf)::value, kMax = decltype(lmax)::value;
+        const auto* y = reinterpret_cast<const C2<T>*>(Fphi);
+        if (phi64) {
+            allow_dynamic_lds(reinterpret_cast<const void*>(&k_ewald_inv<T, double, NF, kMax>), lds);
+            hipLaunchKernelGGL((k_ewald_inv<T, double, NF, kMax>), grid, dim3(NF * kFftThreads), lds, st, G, R, reps,
+                               total, y, phi64);
+        } else {
+            allow_dynamic_lds(reinterpret_cast<const void*>(&k_ewald_inv<T, T, NF, kMax>), lds);
+            hipLaunchKernelGGL((k_ewald_inv<T, T, NF, kMax>), grid, dim3(NF * kFftThreads), lds, st, G, R, reps, total,
+                               y, phi);
+        }
+    };
+    auto forms = [&](auto launch) {
+        if constexpr (sizeof(T) == 4)
+            if (three) {
+                launch(LineLength<3>{}, LineLength<kLineShort>{});
+                return;
+            }
+        if (lines16) launch(LineLength<1>{}, LineLength<kLineShort>{});
+        else launch(LineLength<1>{}, LineLength<kLmax>{});
+    };
+    forms(fwd);
     ewald_contract<T>(G, R, M, Fmu, Fphi, st);
-    const auto* y = reinterpret_cast<const C2<T>*>(Fphi);
-    if (phi64) {
-        allow_dynamic_lds(reinterpret_cast<const void*>(&k_ewald_inv<T, double>), lds);
-        hipLaunchKernelGGL((k_ewald_inv<T, double>), dim3(3 * G.na, R), dim3(kFftThreads), lds, st, G, R, reps,
-                           total, y, phi64);
-    } else {
-        allow_dynamic_lds(reinterpret_cast<const void*>(&k_ewald_inv<T, T>), lds);
-        hipLaunchKernelGGL((k_ewald_inv<T, T>), dim3(3 * G.na, R), dim3(kFftThreads), lds, st, G, R, reps, total, y,
-                           phi);
-    }
+    forms(inv);
     return true;
 }
 
