@@ -497,57 +497,61 @@ bool plan_resident(int na, const std::vector<std::array<int, 3>>& dims, const st
                 ex += w.nlane;
                 K.wg.push_back(w);
             }
-            auto site_of = [&](int e, const std::array<int, 4>& d) {  // bonded site of entry e
-                const int c = e / na;
-                const int x[3] = {c % L[0], c / L[0] % L[1], c / (L[0] * L[1])};
-                int y[3];
-                for (int a = 0; a < 3; a++) y[a] = ((x[a] + d[a]) % L[a] + L[a]) % L[a];
-                return (y[0] + L[0] * (y[1] + L[1] * y[2])) * na + d[3];
-            };
-            // the parts each part reads; the exchange needs it symmetric per site
-            std::vector<std::vector<int>> readers(part.size() > 1 ? ns : 0);
+            std::vector<std::array<int, 3>> fwd(slots.size());  // bond offsets wrapped to 0..L-1
+            for (size_t q = 0; q < slots.size(); q++)
+                for (int a = 0; a < 3; a++) fwd[q][a] = (slots[q][a] % L[a] + L[a]) % L[a];
+            std::vector<int> near;  // bonded sites of the part's entries, slot after slot
+            // the exchange needs every bond to have its reverse
+            for (int i = 0; i < na && part.size() > 1; i++)
+                for (int q = bstart[i]; q < bstart[i + 1]; q++) {
+                    const int j = slots[q][3];
+                    bool back = false;
+                    for (int k = bstart[j]; k < bstart[j + 1] && !back; k++) {
+                        back = slots[k][3] == i;
+                        for (int a = 0; a < 3; a++) back = back && (slots[q][a] + slots[k][a]) % L[a] == 0;
+                    }
+                    if (!back) return false;
+                }
+            std::vector<int> halo, order(ex, -1);  // exchange position -> order in the halo
             for (size_t p = 0; p < part.size(); p++) {
                 ResWg& w = K.wg[p];
-                std::map<int, int> halo;  // exchange position -> order (sorted: neighbouring lanes read neighbouring words)
-                if (part.size() > 1)
-                    for (int e : part[p]) {
-                        const int i = e % na;
-                        for (int q = bstart[i]; q < bstart[i + 1]; q++) {
-                            const int f = site_of(e, slots[q]);
-                            if (who[f] != (int)p) {
-                                halo.emplace(at[f], 0);
-                                readers[f].push_back(e);
-                            }
-                        }
+                halo.clear();
+                near.clear();
+                for (int e : part[p]) {
+                    const int i = e % na, c = e / na, c12 = c / L[0], x1 = c % L[0], x2 = c12 % L[1], x3 = c12 / L[1];
+                    for (int q = bstart[i]; q < bstart[i + 1]; q++) {
+                        int y1 = x1 + fwd[q][0], y2 = x2 + fwd[q][1], y3 = x3 + fwd[q][2];
+                        y1 -= y1 >= L[0] ? L[0] : 0, y2 -= y2 >= L[1] ? L[1] : 0, y3 -= y3 >= L[2] ? L[2] : 0;
+                        const int f = (y1 + L[0] * (y2 + L[1] * y3)) * na + slots[q][3];
+                        near.push_back(f);
+                        if (who[f] == (int)p || order[at[f]] >= 0) continue;
+                        order[at[f]] = 0;
+                        halo.push_back(at[f]);
                     }
-                w.halo0 = (int)out.halo.size();
-                int h = 0;
-                for (auto& kv : halo) {
-                    kv.second = h++;
-                    out.halo.push_back(kv.first);
                 }
-                w.nhalo = h;
+                std::sort(halo.begin(), halo.end());  // neighbouring lanes read neighbouring words
+                w.halo0 = (int)out.halo.size();
+                w.nhalo = (int)halo.size();
+                for (int h = 0; h < w.nhalo; h++) order[halo[h]] = h;
+                out.halo.insert(out.halo.end(), halo.begin(), halo.end());
                 w.nbr0 = (int)out.nbr.size();
                 if (w.nlane + w.nhalo > 65535) return false;
                 out.nbr.resize(out.nbr.size() + (size_t)out.nslot * w.nlane, 0);
+                const int* nf = near.data();
                 for (size_t k = 0; k < part[p].size(); k++) {
-                    const int e = part[p][k], i = e % na;
+                    const int i = part[p][k] % na;
                     for (int q = bstart[i]; q < bstart[i + 1]; q++) {
-                        const int f = site_of(e, slots[q]);
+                        const int f = *nf++;
                         out.nbr[w.nbr0 + (size_t)(q - bstart[i]) * w.nlane + k] =
-                            (unsigned short)(who[f] == (int)p ? at[f] - w.ex0 : w.nlane + halo[at[f]]);
+                            (unsigned short)(who[f] == (int)p ? at[f] - w.ex0 : w.nlane + order[at[f]]);
                     }
                 }
+                for (int x : halo) order[x] = -1;
                 const size_t lds = ((size_t)6 * elem * (w.nlane + w.nhalo) + 2 * (size_t)out.nslot * w.nlane + 15) / 16 * 16;
                 if (lds > lds_max) return false;
                 out.lds = std::max(out.lds, lds);
                 out.threads = std::max(out.threads, part.size() > 1 ? kResThreads : w.nlane);
             }
-            for (size_t f = 0; f < readers.size(); f++)  // f is read by e: e must be read by f
-                for (int e : readers[f]) {
-                    const auto& v = readers[e];
-                    if (std::find(v.begin(), v.end(), (int)f) == v.end()) return false;
-                }
             found = cls.emplace(L, std::move(K)).first;
         }
         const ClassPlan& K = found->second;

@@ -8,8 +8,9 @@
 // The reordering runs here, a chunk at a time, so that a transfer is a
 // packed copy through pinned memory, and the host's only pass over a chunk
 // (widening to doubles) overlaps the next one's copy.  It bounds a transfer
-// at the rate of that pass: 4.2 million FP32 dipoles 30 -> 3.5 ms (a host
-// loop over padded planes from a pageable copy before).  A packed word per
+// at the rate of that pass: 4.2 million FP32 dipoles read into their eight
+// systems 28 -> 6.8 ms (a host loop over padded planes from a pageable copy
+// before).  A packed word per
 // thread keeps the stores coalesced; the three planes' reads of one site run
 // are shared through the cache.
 #include "snh_state.h"
