@@ -87,7 +87,12 @@ typedef struct {
  * Ewald.  One replica of 513 to 28,672 sites without Ewald, on either layout,
  * runs the midpoint steps of a call and calls of several Langevin steps in
  * one cooperative launch (snh_query "cooperative"; SNH_COOP=0 at snh_create
- * launches every stage, SNH_COOP_MAX_SITES lowers the bound). */
+ * launches every stage, SNH_COOP_MAX_SITES lowers the bound).  Its workgroups
+ * wait for each other: where another process keeps some of them off the GPU
+ * for SNH_RES_SPIN polls (2^22), the call is made again from its start by
+ * launches, at the latest when a later call waits, and "cooperative" is 0
+ * from then on; a waiting call returns SNH_ERR_HIP once if
+ * snh_energy_noalloc read the state in between. */
 #define SNH_LAYOUT_AUTO 0
 #define SNH_LAYOUT_GHOST 1
 

@@ -493,6 +493,14 @@ struct SystemImpl final : snh_system {
     unsigned long long* res_ex = nullptr;  // exchanged words of a launch
     int* res_err = nullptr;                // host memory: a wait of some launch timed out
     T* res_sdd = nullptr;                  // where a resident midpoint leaves S'' (the adjoint's recording)
+    T* res_keep = nullptr;                 // the state at the start of the latest call cut into parts
+    struct {                               // the latest resident Langevin call
+        double dt, damping, kT;
+        uint64_t seed, step0;
+        int nsteps;
+    } res_call{};
+    bool res_pending = false;  // it is queued and not yet known to have ended well
+    bool res_read = false;     // snh_energy_noalloc has read its state since
     // Tiled Langevin batches of two or more replicas (no Ewald) step as two
     // replica groups on two streams in anti-phase: one group's corrector
     // (latency-bound) runs beside the other's predictor (VALU-bound).
@@ -629,26 +637,73 @@ struct SystemImpl final : snh_system {
         A.halo = own(dupload(res.halo));
         A.nbr = own(dupload(res.nbr));
         const size_t words = res_words(res, sizeof(T));
-        if (words) res_ex = own(dalloc<unsigned long long>(words));
+        if (words) {
+            res_ex = own(dalloc<unsigned long long>(words));
+            res_keep = own(dalloc<T>(3 * (size_t)interior_sites()));
+        }
         A.ex = res_ex;
         A.res = res_ex ? res_ex + words - 4 * (size_t)res.nres : nullptr;
         A.nslot = res.nslot;
         A.nex = res.nex;
         A.nres = res.nres;
-        A.spin = 1u << 22;
+        A.spin = (unsigned)std::max(0, env_int("SNH_RES_SPIN", 1 << 22));
         SNH_HIP(hipHostMalloc((void**)&res_err, sizeof(int), hipHostMallocDefault));
         *res_err = 0;
         A.err = res_err;
         if (!fail_step) fail_step = own(dalloc<int>(R));
     }
 
-    // After a synchronisation: reports a resident launch whose parts lost
-    // each other (its results are not to be used).
-    void check_resident()
+    // After a synchronisation: true when the parts of a resident call lost
+    // each other (a wait timed out: another process held their compute
+    // units).  The state is then that of the call's start again, and the
+    // handle keeps to launches.
+    bool resident_lost()
     {
-        if (!res_err || *(volatile int*)res_err == 0) return;
+        if (!res_err || *(volatile int*)res_err == 0) return false;
         *res_err = 0;
-        throw Failure{SNH_ERR_HIP, "resident steps: a wait for a neighbouring part timed out"};
+        restore_kept();
+        return true;
+    }
+
+    // The state at the start of the latest resident call; launches from now on.
+    void restore_kept()
+    {
+        coop = false;
+        launch_state_unpack<T>(state_map(), res_keep, 3, 0, interior_sites(), X, st);
+        SNH_HIP(hipGetLastError());
+    }
+
+    // After a synchronisation: makes a Langevin call that was lost again by
+    // launches, which give the same states.  True when it did: what has been
+    // read from the state since the call is to be read again.
+    bool recover()
+    {
+        const bool read = res_read;
+        res_pending = res_read = false;
+        if (!resident_lost()) return false;
+        step_langevin(res_call.dt, res_call.damping, &res_call.kT, nullptr, res_call.seed, res_call.step0,
+                      res_call.nsteps);
+        SNH_HIP(hipStreamSynchronize(st));
+        if (read)
+            throw Failure{SNH_ERR_HIP, "resident steps were made again: an energy queued by snh_energy_noalloc "
+                                       "read them too early"};
+        return true;
+    }
+
+    // Before work that changes the state, or reads it without waiting.
+    void settle()
+    {
+        if (!res_pending) return;
+        SNH_HIP(hipStreamSynchronize(st));
+        recover();
+    }
+
+    // A read of the state that ends synchronised.
+    template <typename F>
+    void settled(F read)
+    {
+        read();
+        if (recover()) read();
     }
 
     void build(const snh_spec& sp)
@@ -1251,7 +1306,6 @@ struct SystemImpl final : snh_system {
             const long long k0 = c * per;
             put(k0, std::min(per, n - k0), xfer.pin[c & 1]);
         }
-        check_resident();
     }
 
     void download_planes(const T* P, int np, double* x)
@@ -1294,6 +1348,7 @@ struct SystemImpl final : snh_system {
         dz_valid = false;
         SNH_REQUIRE(coherent == (N > 0), SNH_ERR_INVALID,
                     coherent ? "coherent states require :SUN mode" : "in :SUN mode set coherent states");
+        settle();
         upload_planes(x, planes, X);
     }
 
@@ -1301,7 +1356,7 @@ struct SystemImpl final : snh_system {
     {
         if (coherent || N == 0) {
             SNH_REQUIRE(!coherent || N > 0, SNH_ERR_INVALID, "coherent states require :SUN mode");
-            download_planes(X, planes, x);
+            settled([&] { download_planes(X, planes, x); });
         } else {
             // dipoles of a coherent state: expected_spin(Z) (Integrators.jl:354), in FP64
             const StateMap M = state_map();
@@ -1545,6 +1600,7 @@ struct SystemImpl final : snh_system {
     void corr_add_sample(double dt, double tol, int max_iters) override
     {
         SNH_REQUIRE(corr.nt > 0, SNH_ERR_INVALID, "sampled correlations are not initialised");
+        settle();
         const int nt = corr.nt, Tsnap = nt / 2 + 1, nobs = corr.nobs;
         const long long ncell = corr.ncell;
         const size_t nsamp = (size_t)nt * nobs * na * ncell;
@@ -1736,6 +1792,7 @@ struct SystemImpl final : snh_system {
             A.cum[p] = c;
         }
         mc_prepare();
+        settle();
         // the sweeps rewrite the state: the expected-dipole planes carried
         // between SU(N) Langevin calls no longer describe it
         dz_valid = false;
@@ -1964,6 +2021,10 @@ struct SystemImpl final : snh_system {
             nz.host = host_noise;
         }
         SNH_HIP(hipStreamSynchronize(st));  // host vectors above are pageable
+        if (recover()) {  // which used the table of scales
+            SNH_HIP(hipMemcpyAsync(nscale, sc.data(), sizeof(T) * R, hipMemcpyHostToDevice, st));
+            SNH_HIP(hipStreamSynchronize(st));
+        }
         const T tdt = (T)dt, tl = (T)damping;
         // SU(N) with bilinear couplings only: the stages exchange expected
         // dipoles (3 planes) instead of kets for the neighbour gather.
@@ -1986,15 +2047,20 @@ struct SystemImpl final : snh_system {
                 nz.step = step0 + (uint64_t)s;
                 hipEvent_t e = tbegin();
                 if (res_ex) launch_res_clear(res_ex, res_words(res, sizeof(T)), conv_iter, fail_step, R, st);
-                const hipError_t le = launch_res_langevin<T>(C, res, res_args, X, nz, tdt, tl,
-                                                             std::min(4096, nsteps - s), st);
+                const hipError_t le = launch_res_langevin<T>(C, res, res_args, X, s == 0 ? res_keep : nullptr, nz,
+                                                             tdt, tl, std::min(4096, nsteps - s), st);
                 tend("dipole_resident", e);
                 if (le == hipSuccess) continue;
                 // parts the device cannot keep resident: launched stages from
-                // now on (same layout, same results)
+                // now on, from the call's start (same layout, same results)
                 (void)hipGetLastError();
-                SNH_REQUIRE(s == 0 && coop, SNH_ERR_HIP, "resident Langevin launch failed");
+                SNH_REQUIRE(coop, SNH_ERR_HIP, "resident Langevin launch failed");
+                if (s > 0) restore_kept();
                 coop = done = false;
+            }
+            if (done && coop) {
+                res_call = {dt, damping, kT[0], seed, step0, nsteps};
+                res_pending = true;
             }
             SNH_HIP(hipGetLastError());
             if (done) return;
@@ -2048,13 +2114,14 @@ struct SystemImpl final : snh_system {
         }
         SNH_HIP(hipMemcpyAsync(atol2, a2.data(), sizeof(double) * R, hipMemcpyHostToDevice, st));
         SNH_HIP(hipStreamSynchronize(st));
+        recover();
         const T tdt = (T)dt, tl = (T)damping;
         if ((persist || coop) && R == 1 && nsteps > 0) {
             // every step iterated to convergence on the device; one host check per call
             hipEvent_t e = tbegin();
             launch_res_clear(res_ex, res_words(res, sizeof(T)), conv_iter, fail_step, R, st);
-            const hipError_t le = launch_res_midpoint<T>(C, res, res_args, X, tdt, tl, atol2, max_iters, nsteps,
-                                                         conv_iter, fail_step, res_sdd, st);
+            const hipError_t le = launch_res_midpoint<T>(C, res, res_args, X, res_keep, tdt, tl, atol2, max_iters,
+                                                         nsteps, conv_iter, fail_step, res_sdd, st);
             tend("midpoint_resident", e);
             if (le != hipSuccess) {
                 // parts the device cannot keep resident: launched sweeps from
@@ -2066,17 +2133,18 @@ struct SystemImpl final : snh_system {
                 SNH_HIP(hipMemcpyAsync(pinned_i, conv_iter, sizeof(int), hipMemcpyDeviceToHost, st));
                 SNH_HIP(hipMemcpyAsync(pinned_i + 1, fail_step, sizeof(int), hipMemcpyDeviceToHost, st));
                 SNH_HIP(hipStreamSynchronize(st));
-                check_resident();
-                if (iters) iters[0] = pinned_i[0];
-                last_iters = pinned_i[0];
-                if (pinned_i[1] >= 0) {
-                    char msg[256];
-                    snprintf(msg, sizeof msg,
-                             "Spherical midpoint method failed to converge to tolerance %g after %d iterations.", tol,
-                             max_iters);
-                    throw Failure{SNH_ERR_NOCONVERGE, msg};
+                if (!resident_lost()) {  // else: launched sweeps, from the call's start
+                    if (iters) iters[0] = pinned_i[0];
+                    last_iters = pinned_i[0];
+                    if (pinned_i[1] >= 0) {
+                        char msg[256];
+                        snprintf(msg, sizeof msg,
+                                 "Spherical midpoint method failed to converge to tolerance %g after %d iterations.",
+                                 tol, max_iters);
+                        throw Failure{SNH_ERR_NOCONVERGE, msg};
+                    }
+                    return;
                 }
-                return;
             }
         }
         ensure_midpoint_buffers();
@@ -2270,6 +2338,7 @@ struct SystemImpl final : snh_system {
     {
         dz_valid = false;
         require_adjoint_support();
+        settle();
         SNH_REQUIRE(nsteps >= 1 && every >= 1, SNH_ERR_INVALID, "nsteps and checkpoint_every must be positive");
         const int ncp = (nsteps + every - 1) / every;
         const size_t bytes = sizeof(T) * planes * (size_t)total;
@@ -2353,6 +2422,7 @@ struct SystemImpl final : snh_system {
             SNH_REQUIRE(rec_n > 0, SNH_ERR_INVALID, "no recorded trajectory: call snh_midpoint_record first");
             SNH_REQUIRE(nparams >= 0 && (nparams == 0 || (params && grad)), SNH_ERR_INVALID, "invalid parameters");
             SNH_REQUIRE(dLdS, SNH_ERR_INVALID, "null loss gradient");
+            settle();
             const size_t np = (size_t)planes * total, bytes = sizeof(T) * np;
             // scratch for this call (freed below)
             std::vector<void*> tmp;
@@ -2479,10 +2549,11 @@ struct SystemImpl final : snh_system {
 
     void energy(double* E) override
     {
-        energy_launch(partial, d_out, true);
-        SNH_HIP(hipMemcpyAsync(pinned, d_out, sizeof(double) * R, hipMemcpyDeviceToHost, st));
-        SNH_HIP(hipStreamSynchronize(st));
-        check_resident();
+        settled([&] {
+            energy_launch(partial, d_out, true);
+            SNH_HIP(hipMemcpyAsync(pinned, d_out, sizeof(double) * R, hipMemcpyDeviceToHost, st));
+            SNH_HIP(hipStreamSynchronize(st));
+        });
         for (int r = 0; r < R; r++) E[r] = pinned[r];
     }
 
@@ -2501,29 +2572,32 @@ struct SystemImpl final : snh_system {
         double* part = noalloc_scratch(dev);
         SNH_REQUIRE(part, SNH_ERR_HIP, "static scratch not resolved on this device");
         energy_launch(part, E_dev, false);
+        res_read = res_pending;
     }
 
     void energy_grad(double* out) override
     {
-        const T* phi = nullptr;
-        if (ewald) {
-            ewald_field(X, phi1);
-            phi = phi1;
-        }
-        if (tiled)
-            launch_tile_grad<T>(C, tp.A, tp.threads, X, phi, Xp, st);
-        else if (N == 0)
-            launch_dipole_grad<T>(C, nblocks, X, phi, Xp, st);
-        else
-            launch_sun_grad<T>(C, nblocks, X, phi, Xp, st);
-        SNH_HIP(hipGetLastError());
-        download_planes(Xp, planes, out);
+        settled([&] {
+            const T* phi = nullptr;
+            if (ewald) {
+                ewald_field(X, phi1);
+                phi = phi1;
+            }
+            if (tiled)
+                launch_tile_grad<T>(C, tp.A, tp.threads, X, phi, Xp, st);
+            else if (N == 0)
+                launch_dipole_grad<T>(C, nblocks, X, phi, Xp, st);
+            else
+                launch_sun_grad<T>(C, nblocks, X, phi, Xp, st);
+            SNH_HIP(hipGetLastError());
+            download_planes(Xp, planes, out);
+        });
     }
 
     void synchronize() override
     {
         SNH_HIP(hipStreamSynchronize(st));
-        check_resident();
+        recover();
     }
 
     void enable_timing(bool on) override

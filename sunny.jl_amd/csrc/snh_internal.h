@@ -254,12 +254,15 @@ bool plan_resident(int na, const std::vector<std::array<int, 3>>& dims, const st
 size_t res_words(const ResPlan& P, size_t elem);  // 8-byte words of ex and res together
 void launch_res_clear(unsigned long long* words, size_t n, int* iters, int* fail, int R, hipStream_t st);
 // Both return the launch status (parts that cannot all be resident are
-// refused).  Sdd (may be null): receives S'' of the last iteration.
+// refused).  keep (may be null): receives the state at the start, [site][3] in
+// the order of the host's states; stored by the lanes that have just loaded
+// it, it takes no time beside the steps (copied before the launch: 7 us of a
+// call at 4096 sites).  Sdd (may be null): receives S'' of the last iteration.
 template <typename T>
-hipError_t launch_res_langevin(const Couplings<T>& C, const ResPlan& P, const ResArgs& A, T* X,
+hipError_t launch_res_langevin(const Couplings<T>& C, const ResPlan& P, const ResArgs& A, T* X, T* keep,
                                const NoiseArgs<T>& nz, T dt, T lambda, int nsteps, hipStream_t st);
 template <typename T>
-hipError_t launch_res_midpoint(const Couplings<T>& C, const ResPlan& P, const ResArgs& A, T* X, T dt, T lambda,
+hipError_t launch_res_midpoint(const Couplings<T>& C, const ResPlan& P, const ResArgs& A, T* X, T* keep, T dt, T lambda,
                                const double* atol2, int max_iters, int nsteps, int* iters_out, int* fail_step,
                                T* Sdd, hipStream_t st);
 

@@ -201,8 +201,9 @@ __device__ __forceinline__ void res_publish(const ResArgs& A, const Part<T>& P, 
     ll_put(p + 2 * kWords<T> * (size_t)A.nex, A.nex, v.z, tag);
 }
 
-// Ends a wait that lasted too long: every thread of the launch stops waiting
-// and the call reports the error.
+// Ends a wait that lasted too long: every thread of the launch stops waiting,
+// the launch runs to its end on whatever it holds, and the host, which kept
+// the state of the call's start, makes the call again stage by stage.
 template <typename T>
 __device__ __forceinline__ bool res_give_up(const ResArgs& A, Part<T>& P, unsigned n)
 {
@@ -255,9 +256,19 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
+// The thread's site of the call's start, in the order of the host's states.
+template <typename T>
+__device__ __forceinline__ void res_keep(const Part<T>& P, T* __restrict__ keep, V3<T> s)
+{
+    T* p = keep + 3 * (size_t)(P.sc.c + P.sc.R.ncell * P.sc.i);
+    p[0] = s.x;
+    p[1] = s.y;
+    p[2] = s.z;
+}
+
 template <typename T, int CH, bool kIso, bool kUni, int NT>
-__global__ __launch_bounds__(NT) void k_res_langevin(Couplings<T> C, ResArgs A, T* X, NoiseArgs<T> nz, T dt,
-                                                     T lambda, int nsteps)
+__global__ __launch_bounds__(NT) void k_res_langevin(Couplings<T> C, ResArgs A, T* X, T* __restrict__ keep,
+                                                     NoiseArgs<T> nz, T dt, T lambda, int nsteps)
 {
     Part<T> P = res_part<T, kUni>(C, A);
     T* const b0 = P.buf;                 // S
@@ -269,6 +280,7 @@ __global__ __launch_bounds__(NT) void k_res_langevin(Couplings<T> C, ResArgs A, 
     V3<T> s = {0, 0, 0}, xi = {0, 0, 0};
     if (P.own) {
         s = planes(X, C.total)(P.sc.g);
+        if (keep) res_keep(P, keep, s);
         lds_put(b0, P.nsite, P.t, s);
         if (noisy) xi = dipole_noise(nz, P.sc.r, site, P.sc.g);
     }
@@ -334,8 +346,8 @@ __device__ __forceinline__ void res_residual(const ResArgs& A, Part<T>& P, unsig
 }
 
 template <typename T, int CH, bool kIso, bool kUni, int NT>
-__global__ __launch_bounds__(NT) void k_res_midpoint(Couplings<T> C, ResArgs A, T* X, T dt, T lambda,
-                                                     const double* __restrict__ atol2, int max_iters, int nsteps,
+__global__ __launch_bounds__(NT) void k_res_midpoint(Couplings<T> C, ResArgs A, T* X, T* __restrict__ keep, T dt,
+                                                     T lambda, const double* __restrict__ atol2, int max_iters, int nsteps,
                                                      int* __restrict__ iters_out, int* __restrict__ fail_step,
                                                      T* Sdd)
 {
@@ -346,7 +358,10 @@ __global__ __launch_bounds__(NT) void k_res_midpoint(Couplings<T> C, ResArgs A, 
     const bool parts = P.w.nresr != 0;  // several workgroups share the replica
     const int nwave = P.w.nlane / 64;
     V3<T> s = {0, 0, 0}, prev = {0, 0, 0};
-    if (P.own) s = planes(X, C.total)(P.sc.g);
+    if (P.own) {
+        s = planes(X, C.total)(P.sc.g);
+        if (keep) res_keep(P, keep, s);
+    }
     unsigned tag = 0, rtag = 0;
     int p = 0, it = 0, failed = -1;
     __syncthreads();  // the bond table
@@ -635,32 +650,32 @@ void launch_res_clear(unsigned long long* words, size_t n, int* iters, int* fail
 }
 
 template <typename T>
-hipError_t launch_res_langevin(const Couplings<T>& C, const ResPlan& P, const ResArgs& A, T* X,
+hipError_t launch_res_langevin(const Couplings<T>& C, const ResPlan& P, const ResArgs& A, T* X, T* keep,
                                const NoiseArgs<T>& nz, T dt, T lambda, int nsteps, hipStream_t st)
 {
     Couplings<T> c = C;
     ResArgs a = A;
     NoiseArgs<T> z = nz;
-    void* args[] = {&c, &a, &X, &z, &dt, &lambda, &nsteps};
+    void* args[] = {&c, &a, &X, &keep, &z, &dt, &lambda, &nsteps};
     return launch_res_forms<T, true>(C, P, args, st);
 }
 
 template <typename T>
-hipError_t launch_res_midpoint(const Couplings<T>& C, const ResPlan& P, const ResArgs& A, T* X, T dt, T lambda,
+hipError_t launch_res_midpoint(const Couplings<T>& C, const ResPlan& P, const ResArgs& A, T* X, T* keep, T dt, T lambda,
                                const double* atol2, int max_iters, int nsteps, int* iters_out, int* fail_step,
                                T* Sdd, hipStream_t st)
 {
     Couplings<T> c = C;
     ResArgs a = A;
-    void* args[] = {&c, &a, &X, &dt, &lambda, &atol2, &max_iters, &nsteps, &iters_out, &fail_step, &Sdd};
+    void* args[] = {&c, &a, &X, &keep, &dt, &lambda, &atol2, &max_iters, &nsteps, &iters_out, &fail_step, &Sdd};
     return launch_res_forms<T, false>(C, P, args, st);
 }
 
 #define SNH_INST(T)                                                                                             \
-    template hipError_t launch_res_langevin<T>(const Couplings<T>&, const ResPlan&, const ResArgs&, T*,         \
+    template hipError_t launch_res_langevin<T>(const Couplings<T>&, const ResPlan&, const ResArgs&, T*, T*,     \
                                                const NoiseArgs<T>&, T, T, int, hipStream_t);                    \
-    template hipError_t launch_res_midpoint<T>(const Couplings<T>&, const ResPlan&, const ResArgs&, T*, T, T,   \
-                                               const double*, int, int, int*, int*, T*, hipStream_t);
+    template hipError_t launch_res_midpoint<T>(const Couplings<T>&, const ResPlan&, const ResArgs&, T*, T*, T,  \
+                                               T, const double*, int, int, int*, int*, T*, hipStream_t);
 SNH_INST(float)
 SNH_INST(double)
 

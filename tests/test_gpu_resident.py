@@ -97,3 +97,97 @@ def test_resident_steps_match_launches(kind, dims, precision, layout, monkeypatc
     ia, ib = sh.step_(a, mid, nsteps=7), sh.step_(b, mid, nsteps=7)
     assert abs(int(ia[0]) - int(ib[0])) <= 1
     assert rel_err(a.dipoles_flat(), b.dipoles_flat(), scale=kap) <= TOL[precision] + mid.tol
+
+
+def next_calls():
+    """What a program may do after a Langevin call: reads of the state, and
+    everything that changes it."""
+    lang, mid = sh.Langevin(0.03, damping=0.2, kT=0.7), sh.ImplicitMidpoint(0.02, damping=0.1)
+    sampler = sh.LocalSampler(kT=0.4, nsweeps=1.5)
+    return {
+        "spins": lambda s: None,
+        "energy": sh.energy,
+        "gradient": sh.energy_grad_dipoles,
+        "synchronize": lambda s: s._device().call("snh_synchronize"),
+        "steps": lambda s: sh.step_(s, lang, nsteps=3),
+        "midpoint": lambda s: sh.step_(s, mid, nsteps=2),
+        "sampler": lambda s: sh.step_(s, sampler),
+    }
+
+
+@pytest.mark.parametrize("after", list(next_calls()))
+def test_lost_parts_leave_the_launched_result(after, monkeypatch):
+    """Parts that give up waiting (here at the first word that is not there
+    yet) must not cost the state: the call is made again by launches, whatever
+    comes next, and the handle keeps to them."""
+    announce(f"lost Langevin parts, then {after}")
+
+    def run(coop, spin):
+        monkeypatch.setenv("SNH_COOP", coop)
+        monkeypatch.setenv("SNH_RES_SPIN", spin)
+        s = sh.workloads.cubic_model(L=16, seed=7, precision=64)
+        s.layout = 1
+        assert s._device().query("cooperative") == int(coop)
+        sh.step_(s, sh.Langevin(0.05, damping=0.1, kT=0.5), nsteps=40)
+        out = next_calls()[after](s)
+        first = s.dipoles_flat()
+        s._dev_dirty = True
+        np.testing.assert_array_equal(s.dipoles_flat(), first)  # a second read
+        return s, out, first
+
+    a, oa, Sa = run("1", "0")
+    b, ob, Sb = run("0", "0")
+    assert a._device().query("cooperative") == 0
+    np.testing.assert_array_equal(Sa, Sb)
+    if ob is not None:
+        np.testing.assert_array_equal(oa, ob)
+    a.set_state_flat(dip=Sa[::-1].copy())  # and a new state is taken as ever
+    sh.energy(a)
+    a._dev_dirty = True
+    np.testing.assert_array_equal(a.dipoles_flat(), Sa[::-1])
+
+
+def test_lost_midpoint_parts_leave_the_launched_result(monkeypatch):
+    announce("lost midpoint parts")
+
+    def make(coop):
+        monkeypatch.setenv("SNH_COOP", coop)
+        monkeypatch.setenv("SNH_RES_SPIN", "0")
+        s = sh.workloads.cubic_model(L=16, seed=7, precision=64)
+        s.layout = 1
+        s._device()
+        return s
+
+    a, b = make("1"), make("0")
+    mid = sh.ImplicitMidpoint(0.02, damping=0.1)
+    np.testing.assert_array_equal(sh.step_(a, mid, nsteps=5), sh.step_(b, mid, nsteps=5))
+    assert a._device().query("cooperative") == 0
+    np.testing.assert_array_equal(a.dipoles_flat(), b.dipoles_flat())
+    # a trajectory's recording loses its first step and goes on by launches
+    w = np.arange(3.0 * a.nsites).reshape(-1, 3)
+    grads = [sh.midpoint_gradient(s, sh.ImplicitMidpoint(0.02), 4, [], lambda S: (float((w * S).sum()), w))
+             for s in (make("1"), make("0"))]
+    for x, y in zip(*grads):
+        np.testing.assert_array_equal(x, y)
+
+
+def test_energy_read_from_lost_parts_is_reported(monkeypatch):
+    """An energy queued without waiting reads a lost call's spins before the
+    call is made again: the next waiting call says so, once, and the state is
+    the launched one."""
+    announce("lost parts, energy without waiting")
+    from test_zz_no_alloc import noalloc_energy
+
+    def make(coop):
+        monkeypatch.setenv("SNH_COOP", coop)
+        monkeypatch.setenv("SNH_RES_SPIN", "0")
+        s = sh.workloads.cubic_model(L=16, seed=7, precision=64)
+        s.layout = 1
+        sh.step_(s, sh.Langevin(0.05, damping=0.1, kT=0.5), nsteps=40)
+        return s
+
+    a, b = make("1"), make("0")
+    with pytest.raises(RuntimeError, match="made again"):
+        noalloc_energy(a)
+    np.testing.assert_array_equal(noalloc_energy(a), noalloc_energy(b))
+    np.testing.assert_array_equal(a.dipoles_flat(), b.dipoles_flat())
