@@ -492,7 +492,6 @@ struct SystemImpl final : snh_system {
     ResArgs res_args{};
     unsigned long long* res_ex = nullptr;  // exchanged words of a launch
     int* res_err = nullptr;                // host memory: a wait of some launch timed out
-    T* res_sdd = nullptr;                  // where a resident midpoint leaves S'' (the adjoint's recording)
     T* res_keep = nullptr;                 // the state at the start of the latest call cut into parts
     struct {                               // the latest resident Langevin call
         double dt, damping, kT;
@@ -2102,6 +2101,12 @@ struct SystemImpl final : snh_system {
 
     void step_midpoint(double dt, double damping, double tol, int max_iters, int nsteps, int* iters) override
     {
+        midpoint_steps(dt, damping, tol, max_iters, nsteps, iters, nullptr);
+    }
+
+    // Sdd (may be null): where a resident call leaves S'' of its last iteration.
+    void midpoint_steps(double dt, double damping, double tol, int max_iters, int nsteps, int* iters, T* Sdd)
+    {
         dz_valid = false;
         SNH_REQUIRE(std::isfinite(dt) && dt > 0, SNH_ERR_INVALID, "Select positive dt");
         SNH_REQUIRE(damping >= 0, SNH_ERR_INVALID, "Select nonnegative damping");
@@ -2121,7 +2126,7 @@ struct SystemImpl final : snh_system {
             hipEvent_t e = tbegin();
             launch_res_clear(res_ex, res_words(res, sizeof(T)), conv_iter, fail_step, R, st);
             const hipError_t le = launch_res_midpoint<T>(C, res, res_args, X, res_keep, tdt, tl, atol2, max_iters,
-                                                         nsteps, conv_iter, fail_step, res_sdd, st);
+                                                         nsteps, conv_iter, fail_step, Sdd, st);
             tend("midpoint_resident", e);
             if (le != hipSuccess) {
                 // parts the device cannot keep resident: launched sweeps from
@@ -2327,9 +2332,7 @@ struct SystemImpl final : snh_system {
     T* midpoint_one(double dt, double tol, int max_iters, int* it_out)
     {
         ensure_midpoint_buffers();
-        res_sdd = B1;  // a resident launch writes S'' there
-        step_midpoint(dt, 0.0, tol, max_iters, 1, it_out);
-        res_sdd = nullptr;
+        midpoint_steps(dt, 0.0, tol, max_iters, 1, it_out, B1);  // a resident launch writes S'' there
         // launched sweeps: S'' of iteration m lives in B1 for odd m, B2 for even m
         return persist || coop || *it_out % 2 == 1 ? B1 : B2;
     }
