@@ -350,7 +350,10 @@ int snh_autotune(snh_system *sys, int32_t candidates, int32_t launches, double *
  * and one workgroup per in-plane wavevector for the third axis and the
  * contraction; groups of at most 2 replicas, SNH_EWALD_SLAB=0 never, =2 up
  * to 4), "corr_fft_lib" (1 when the
- * sampled correlations' lattice transform uses a hipFFT plan). */
+ * sampled correlations' lattice transform uses a hipFFT plan), "persistent"
+ * and "cooperative" (1 when calls may step resident: replicas of one
+ * workgroup each, or one replica cut into parts), "resident_calls" (calls
+ * that did). */
 int snh_query(snh_system *sys, const char *key, int64_t *value);
 
 #ifdef __cplusplus

@@ -499,6 +499,7 @@ struct SystemImpl final : snh_system {
         int nsteps;
     } res_call{};
     bool res_pending = false;  // it is queued and not yet known to have ended well
+    int64_t res_calls = 0;     // calls stepped resident
     bool res_read = false;     // snh_energy_noalloc has read its state since
     // Tiled Langevin batches of two or more replicas (no Ewald) step as two
     // replica groups on two streams in anti-phase: one group's corrector
@@ -2039,7 +2040,7 @@ struct SystemImpl final : snh_system {
             dz_valid = true;
         }
         if (persist || (coop && graph_steps == 0 && !timer.enabled &&
-                         nsteps >= res_min_steps(replica_sites(0)))) {
+                         nsteps >= res_min_steps(replica_sites(0), res.nslot, tiled))) {
             // chunks bound the length of one launch
             bool done = true;
             for (int s = 0; s < nsteps && done; s += 4096) {
@@ -2057,6 +2058,7 @@ struct SystemImpl final : snh_system {
                 if (s > 0) restore_kept();
                 coop = done = false;
             }
+            res_calls += done;
             if (done && coop) {
                 res_call = {dt, damping, kT[0], seed, step0, nsteps};
                 res_pending = true;
@@ -2138,6 +2140,7 @@ struct SystemImpl final : snh_system {
                 SNH_HIP(hipMemcpyAsync(pinned_i, conv_iter, sizeof(int), hipMemcpyDeviceToHost, st));
                 SNH_HIP(hipMemcpyAsync(pinned_i + 1, fail_step, sizeof(int), hipMemcpyDeviceToHost, st));
                 SNH_HIP(hipStreamSynchronize(st));
+                ++res_calls;
                 if (!resident_lost()) {  // else: launched sweeps, from the call's start
                     if (iters) iters[0] = pinned_i[0];
                     last_iters = pinned_i[0];
@@ -2644,6 +2647,7 @@ struct SystemImpl final : snh_system {
         if (key == "graph_steps") return graph_steps;
         if (key == "persistent") return persist ? 1 : 0;
         if (key == "cooperative") return coop ? 1 : 0;
+        if (key == "resident_calls") return res_calls;
         if (key == "graph_live") return graph_exec ? 1 : 0;
         if (key == "pair_split") return pair_split;
         if (key == "pair_on") return pair_on ? 1 : 0;

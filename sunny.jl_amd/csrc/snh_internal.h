@@ -209,11 +209,22 @@ constexpr int kResOneWg = 512;
 constexpr int kResThreads = 256;
 constexpr int kResMaxSites = 28672;
 constexpr int kResGhostSites = 8192;  // up to here AUTO takes the ghost layout
-// Langevin steps of a call from which parts pay (a cooperative launch costs
-// about 20 us more than a plain one): calls of 4 steps 17.1 against 17.7 us a
-// step at 4096 sites, 20.1 / 20.4 at 8192, but 18.2 / 17.7 at 21,952 and 24.9 /
-// 20.6 at 27,648; calls of 8 steps 10.6 / 14.3, 14.1 / 17.0, 12.0 / 14.4, 18.5 / 18.2.
-constexpr int res_min_steps(long long sites) { return 4 + (int)(sites / 8192); }
+// Langevin steps of a call from which parts pay: a cooperative launch costs
+// about 20 us more than plain ones, and a resident step gains the less the
+// more sites and bond slots its parts share a compute unit with.  us per call,
+// resident / launched, where the two are about equal and the rule's count:
+// tiled layout (slower launches), FP32: cubic 30^3 64/63 at 3, pyrochlore
+// 12^3 x 16 67/68 at 2: 3.  Ghost layout, FP64: cubic 16^3 67/68 at 4, 71/78 at
+// 5; 25^3 80/78 at 5, 85/88 at 6; 30^3 89/88 at 6, 100/110 at 8; pyrochlore 4^3
+// 78/77 at 5; 8^3 89/90 at 5; 10^3 105/105 at 6; 11^3 182/183 at 12; 12^3
+// 243/235 at 16, 337/340 at 24.  Both forms give the same states bit for bit,
+// so that a run does not depend on how it is cut into calls.
+constexpr int res_min_steps(long long sites, int nslot, bool tiled)
+{
+    if (tiled) return 3;
+    const long long over = sites * nslot - 262144;  // bond slots of a stage
+    return 5 + (int)(sites / 8192) + (over > 0 ? (int)(over / 16384) : 0);
+}
 struct ResWg {
     int r;                  // replica
     int first;              // the replica's first part (reports iterations)

@@ -3,8 +3,8 @@ launch per stage on the same layout: sizes around one workgroup and around
 the largest exchange, ragged parts, axes shorter than a bond, many
 sublattices, and every kind of bond and onsite term.
 
-Both run the same per-site arithmetic.  Seven Langevin or midpoint steps
-round about 7 x 20 times; with the spread of one rounding over the steps
+Both run the same per-site arithmetic.  Seven Langevin or midpoint steps (or
+eight, with the same bound, of the largest replicas) round about 7 x 20 times; with the spread of one rounding over the steps
 (at most tenfold) that is 7 x 20 x 10 x 2^-53 = 1.6e-13 in FP64 and 8e-5 in
 FP32, relative to |S|.
 """
@@ -81,22 +81,100 @@ def test_resident_steps_match_launches(kind, dims, precision, layout, monkeypatc
         assert h.query("persistent") + h.query("cooperative") == int(on)
         return s
 
+    def resident(calls):
+        h = a._device()
+        assert h.query("resident_calls") == calls and h.query("persistent") + h.query("cooperative") == 1
+        assert b._device().query("resident_calls") == 0
+
     a, b = handle("1"), handle("0")
     kap = float(np.max(a.kappas))
     lang = sh.Langevin(0.02 / kap, damping=0.1, kT=0.4)
-    sh.step_(a, lang, nsteps=7)
-    sh.step_(b, lang, nsteps=7)
+    n = 7 if a.nsites < 20000 else 8  # from which the largest replicas step resident
+    sh.step_(a, lang, nsteps=n)
+    sh.step_(b, lang, nsteps=n)
     assert np.all(np.isfinite(b.dipoles_flat()))
     assert rel_err(a.dipoles_flat(), b.dipoles_flat(), scale=kap) <= TOL[precision]
     # the noise goes on where the call before ended
-    sh.step_(a, lang, nsteps=5)
-    sh.step_(b, lang, nsteps=5)
+    sh.step_(a, lang, nsteps=n)
+    sh.step_(b, lang, nsteps=n)
     assert rel_err(a.dipoles_flat(), b.dipoles_flat(), scale=kap) <= 2 * TOL[precision]
+    resident(2)
     b.set_state_flat(dip=a.dipoles_flat())
     mid = sh.ImplicitMidpoint(0.01 / kap, damping=0.05, tol=1e-12 if precision == 64 else 1e-5)
     ia, ib = sh.step_(a, mid, nsteps=7), sh.step_(b, mid, nsteps=7)
     assert abs(int(ia[0]) - int(ib[0])) <= 1
     assert rel_err(a.dipoles_flat(), b.dipoles_flat(), scale=kap) <= TOL[precision] + mid.tol
+    resident(3)
+
+
+@pytest.mark.parametrize("kind,dims,precision,layout,least", [
+    ("cubic", (27, 19, 1), 64, 1, 5),       # the smallest that is cut
+    ("cubic", (16, 16, 32), 32, 1, 6),
+    ("cubic", (27, 29, 31), 32, 0, 3),      # tiled layout
+    ("cubic", (28, 32, 32), 64, 1, 8),      # 28672 sites: the most
+    ("pyrochlore", (4, 3, 5), 64, 1, 5),
+    ("pyrochlore", (12, 12, 12), 64, 1, 22),  # 18 bonds a site: a resident step gains little
+    ("pyrochlore", (12, 11, 12), 32, 0, 3),
+    ("general", (11, 9, 8), 64, 1, 5),
+    ("general", (11, 9, 8), 32, 1, 5),
+    ("inhomogeneous", (9, 9, 9), 32, 1, 5),
+])
+def test_langevin_calls_may_be_split_anywhere(kind, dims, precision, layout, least, monkeypatch):
+    """Calls of few steps are launched, longer ones resident, and all calls
+    launched while kernels are timed: the states are the same bit for bit
+    however a run is cut into calls."""
+    announce(f"split calls {kind} {dims} fp{precision} layout {layout}")
+    monkeypatch.setenv("SNH_COOP", "1")
+
+    def run(calls, timed=False, kT=0.4):
+        s = build(kind, dims, precision)
+        s.layout = layout
+        h = s._device()
+        assert h.query("layout") == layout
+        kap = float(np.max(s.kappas))
+        h.call("snh_enable_timing", int(timed))
+        for n in calls:
+            before = h.query("resident_calls")
+            sh.step_(s, sh.Langevin(0.02 / kap, damping=0.1, kT=kT), nsteps=n)
+            assert h.query("resident_calls") - before == int(n >= least and not timed)
+        S = s.dipoles_flat()
+        assert h.query("cooperative") == 1
+        return S
+
+    n = 2 * least + 3
+    whole = run([n])
+    assert np.all(np.isfinite(whole))
+    np.testing.assert_array_equal(run([1, least, 1, least - 1, 2]), whole)
+    np.testing.assert_array_equal(run([least - 1, n + 1 - least]), whole)
+    np.testing.assert_array_equal(run([n], timed=True), whole)
+    np.testing.assert_array_equal(run([n], kT=0.0), run([1] * n, kT=0.0))  # and without noise
+
+
+@pytest.mark.parametrize("dims", [(6, 7, 9), (9, 10, 7)])  # one part; several
+def test_calls_longer_than_a_launch(dims, monkeypatch):
+    """4096 steps are one launch, the rest of the call the next: the noise and
+    the exchanged words go on across them."""
+    announce(f"9000 steps in a call {dims}")
+    monkeypatch.setenv("SNH_PERSIST", "1")
+    monkeypatch.setenv("SNH_COOP", "1")
+    lang = sh.Langevin(0.05, damping=0.1, kT=0.4)
+    out = []
+    for calls in ([9000], [4096, 4096, 808], [5000, 4000]):
+        s = build("cubic", dims, 64)
+        s.layout = 1
+        for n in calls:
+            sh.step_(s, lang, nsteps=n)
+        out.append(s.dipoles_flat())
+        assert s._device().query("resident_calls") == len(calls)
+        assert s._device().query("persistent") + s._device().query("cooperative") == 1
+    np.testing.assert_array_equal(out[1], out[0])
+    np.testing.assert_array_equal(out[2], out[0])
+    monkeypatch.setenv("SNH_PERSIST", "0")
+    monkeypatch.setenv("SNH_COOP", "0")
+    s = build("cubic", dims, 64)
+    s.layout = 1
+    sh.step_(s, lang, nsteps=9000)
+    np.testing.assert_array_equal(s.dipoles_flat(), out[0])
 
 
 def next_calls():
