@@ -47,10 +47,11 @@ namespace snh {
 
 constexpr int kFftThreads = 256;
 constexpr int kSpecKB = 16;  // wavevectors per spectrum block (128-byte runs in FP32)
-// The transforms take three fields a workgroup up to this LDS (two workgroups
-// per CU) and from this count of workgroups (sublattices x replicas).
-constexpr size_t kFieldsLds3 = 80 * 1024;
+// Workgroups (sublattices x replicas) from which the transforms of axes up to
+// kLineShort take three fields a workgroup: one for each compute unit.
 constexpr int kFieldsMin3 = 256;
+static_assert(((size_t)3 * (kLineShort / 2 + 1) * kLineShort * kLineShort + 3 * kLmax) * 2 * sizeof(float) <= 80 * 1024,
+              "two workgroups of three FP32 fields fit the LDS of a compute unit");
 
 // ---------------------------------------------------------------------------
 // One workgroup transforms one field.  Dynamic LDS: spectrum [nk] complex,
@@ -1036,11 +1037,10 @@ bool launch_ewald_field(const EwaldGeom& G, int R, const ReplicaInfo* reps, uint
         }
         return true;
     }
-    // three fields a workgroup (FP32) where two such workgroups fit a CU's
-    // LDS and there are workgroups for most CUs
+    // three fields a workgroup (FP32 lines in registers) where there is such a
+    // workgroup for every CU (figures at k_ewald_fwd)
     const bool lines16 = std::max({G.L1, G.L2, G.L3}) <= kLineShort;
-    const bool three = sizeof(T) == 4 && lines16 && G.na * R >= kFieldsMin3 &&
-                       ewald_fields_lds_bytes(G, 3, sizeof(T)) <= kFieldsLds3;
+    const bool three = sizeof(T) == 4 && lines16 && G.na * R >= kFieldsMin3;
     const size_t lds = ewald_fields_lds_bytes(G, three ? 3 : 1, sizeof(T));
     const dim3 grid((unsigned)(three ? G.na : 3 * G.na), (unsigned)R);
     auto fwd = [&](auto nf, auto lmax) {

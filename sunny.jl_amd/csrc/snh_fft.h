@@ -220,8 +220,9 @@ __device__ __forceinline__ void lines_c2c(C2<T>* buf, int n, Base base, int stri
         for (int l = threadIdx.x; l < n; l += blockDim.x) line_c2c_any<T>(buf + base(l), 0, stride, L, tw);
 }
 
-// Real lines in(l)[0..L) -> half spectra out(l)[0..L/2] (forward); a line may
-// share its storage with its spectrum (direct DFT lengths: not).
+// Real lines in(l)[0..L) -> half spectra out(l)[0..L/2] (forward).  A line may
+// share its storage with its spectrum: in every form a thread holds all
+// outputs of its line until it has read the last input.
 template <int kMax, typename T, typename In, typename Out>
 __device__ __forceinline__ void lines_r2c(int n, In in, Out out, int L, const C2<T>* tw)
 {
@@ -266,7 +267,7 @@ __device__ __forceinline__ void lines_r2c(int n, In in, Out out, int L, const C2
 // Half spectra in(l)[0..L/2] -> real lines out(l)[0..L) (backward, unscaled):
 // the real part of the inverse transform of the Hermitian extension
 // X[L-k] = conj(X[k]); imaginary parts of X[0] and X[L/2] drop out, as c2r.
-// A line may share its storage with its spectrum.
+// A line may share its storage with its spectrum, as above.
 template <int kMax, typename T, typename In, typename Out>
 __device__ __forceinline__ void lines_c2r(int n, In in, Out out, int L, const C2<T>* tw)
 {

@@ -38,7 +38,7 @@ def test_line_lengths(L, precision, tol, monkeypatch):
             assert abs(sh.energy(s) - o.energy(S)) <= tol * np.abs(g * S).sum()
 
 
-@pytest.mark.parametrize("dims", [(5, 3, 4), (8, 7, 2)])
+@pytest.mark.parametrize("dims", [(5, 3, 4), (8, 7, 2), (16, 3, 2), (3, 2, 16)])
 def test_three_fields_a_workgroup(dims):
     announce(f"three fields {dims}")
     one = sh.workloads.pyrochlore_model(dims=dims, J1=0.05, J2=0.0, A=0.0, s=3.5, seed=3, precision=32, dipolar=True)
@@ -52,3 +52,28 @@ def test_three_fields_a_workgroup(dims):
     n = one.nsites
     for r in (0, 7, 15):
         assert rel_err(g[r * n:(r + 1) * n], O.Oracle(one.spec()).grad(systems[r].dipoles_flat())) <= 2e-5
+
+
+@pytest.mark.parametrize("dims", [(5, 3, 4), (2, 16, 2)])
+def test_three_fields_with_the_potential_in_fp64(dims):
+    """The batch's Metropolis trials refresh their FP64 potential by the same
+    transforms after every 512 trials: the energy changes they add up are the
+    oracle's energy differences, to 2e-5 of a full turn in the largest local
+    field for each trial."""
+    announce(f"three fields, FP64 potential {dims}")
+    one = sh.workloads.pyrochlore_model(dims=dims, J1=0.05, J2=0.0, A=0.0, s=3.5, seed=5, precision=32, dipolar=True)
+    systems = [sh.clone_system(one, seed=r) for r in range(16)]
+    for s in systems:
+        sh.randomize_spins_(s)
+    o = O.Oracle(one.spec())
+    before = [s.dipoles_flat() for s in systems]
+    b = sh.ReplicaBatch(systems, precision=32)
+    sampler = sh.LocalSampler(kT=2.0, nsweeps=1.0)
+    sh.step_(b, sampler)
+    b.sync_to_systems()
+    assert one.nsites > 512
+    for r in (0, 7, 15):
+        after = systems[r].dipoles_flat()
+        turn = 2 * 3.5 * np.max(np.linalg.norm(o.grad(before[r]), axis=1))
+        assert abs(sampler.dE[r] - (o.energy(after) - o.energy(before[r]))) <= 2e-5 * one.nsites * turn
+        assert np.count_nonzero(np.any(after != before[r], axis=1)) > one.nsites // 10
