@@ -344,7 +344,7 @@ def bench_corr(args):
     sh.add_sample_(sc, s)
     h.call("snh_synchronize")
     t1 = time.perf_counter()
-    traj_ms, _ = kernel_time(h, "midpoint_iter")
+    traj_ms = sum(kernel_time(h, f)[0] for f in ("midpoint_iter", "midpoint_resident"))
     h.call("snh_enable_timing", 0)
     nsteps = sc.measperiod * (sc.n_all_omega // 2)
     # host restatement of accum_sample! on the same sizes (zero trajectory)

@@ -218,7 +218,8 @@ int snh_midpoint_adjoint(snh_system *sys, int32_t nparams, const snh_spec *param
 /* Diagnostics with no counterpart in the reference: per-kernel timing by HIP
  * events recorded on the handle's stream around every launch of a kernel
  * family ("dipole_predict", "dipole_correct", "sun_predict", "sun_correct",
- * "midpoint_iter", "ewald_field").  enable = 0 stops recording and clears
+ * "midpoint_iter", "dipole_resident", "midpoint_resident", "ewald_field",
+ * "local_color", "local_ewald").  enable = 0 stops recording and clears
  * the totals.  snh_kernel_time synchronises and reports the summed
  * milliseconds and the number of launches recorded since enabling. */
 int snh_enable_timing(snh_system *sys, int32_t enable);

@@ -17,7 +17,9 @@
 // iteration plus one per step.
 //
 // A published dipole is split into 8-byte words, each 4 data bytes and the
-// 4-byte round number, stored and loaded with relaxed agent-scope atomics.
+// 4-byte round number, stored and loaded with relaxed agent-scope atomics:
+// the flag-with-the-data words that collective libraries publish as their
+// low-latency (LL) protocol, hence the prefix ll_.
 // A reader polls until every word carries its round: the data needs no
 // fence, no flag and no cache write-back, and one store-to-load latency
 // across the XCDs is all a round costs, against a release, an arrival
@@ -157,7 +159,8 @@ __device__ __forceinline__ Part<T> res_part(const Couplings<T>& C, const ResArgs
 // are those of local_field.  An isotropic bond is one fused multiply-add per
 // component in the launched Heun stages and a product and a sum in the
 // launched midpoint sweeps (whose general form the compiler cannot fuse);
-// kFused follows suit, so that FP64 states agree bitwise.
+// kFused follows suit, so that Langevin states agree bitwise, and midpoint
+// ones in FP64.
 template <typename T, int CH, bool kIso, bool kFused>
 __device__ __forceinline__ V3<T> res_field(const Couplings<T>& C, const Part<T>& P, const T* b, V3<T> s)
 {

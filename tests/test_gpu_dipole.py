@@ -242,9 +242,9 @@ def test_autotune_keeps_results():
 
 
 def test_cooperative_midpoint_matches_launches(monkeypatch):
-    """One :dipole replica of 512 < sites <= 8192 without Ewald steps the
-    midpoint in one cooperative launch, a grid barrier per fixed-point
-    iteration: iteration counts and states equal, bitwise, the launched
+    """One :dipole replica of 512 < sites <= 28,672 without Ewald steps the
+    midpoint in one cooperative launch, an exchange of border sites per
+    fixed-point iteration: iteration counts and states equal, bitwise, the launched
     sweeps on the same ghost layout, and the oracle's midpoint steps; a step
     that does not converge raises the reference's error and keeps the state
     of the previous step."""
@@ -270,7 +270,7 @@ def test_cooperative_midpoint_matches_launches(monkeypatch):
         for _ in range(n):
             S, _ = o.step_midpoint(S=S, dt=dt, damping=0.1)
     assert rel_err(a.dipoles_flat(), S, scale=1.0) <= 1e-11
-    # a pyrochlore replica of 8192 sites (32 workgroups, 18 bonds per site)
+    # a pyrochlore replica of 8192 sites (128 parts, 18 bonds per site)
     monkeypatch.setenv("SNH_COOP", "1")
     p = sh.workloads.pyrochlore_model(L=8, seed=72, precision=64)
     assert p._device().query("cooperative") == 1
@@ -290,8 +290,8 @@ def test_cooperative_midpoint_matches_launches(monkeypatch):
 
 
 def test_persistent_small_replicas_match_launches(monkeypatch):
-    """Small :dipole replicas on the ghost layout step in one persistent
-    workgroup per replica; the results equal the per-stage launches (same
+    """Small :dipole replicas on the ghost layout step in one workgroup per
+    replica and launch; the results equal the per-stage launches (same
     per-site arithmetic) and the oracle."""
     dims = [(6, 6, 6), (4, 5, 3), (8, 2, 4)]
 

@@ -43,7 +43,7 @@ def test_graph_replays_match_eager(kind, monkeypatch):
     announce(f"graph vs eager {kind}")
     # graphs are opt-in, read at handle creation; they replay the per-stage
     # launches, which small ghost-layout replicas would otherwise replace by
-    # the persistent kernel
+    # resident steps
     monkeypatch.setenv("SNH_PERSIST", "0")
     monkeypatch.setenv("SNH_GRAPH_STEPS", "8")
     a = twins(kind)[0]
