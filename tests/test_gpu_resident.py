@@ -177,6 +177,40 @@ def test_calls_longer_than_a_launch(dims, monkeypatch):
     np.testing.assert_array_equal(s.dipoles_flat(), out[0])
 
 
+def test_handles_of_several_threads():
+    """Four replicas of 432 parts each, more than the device holds side by
+    side, step on four threads: every launch finds its parts resident, and the
+    states are those of one thread."""
+    import threading
+
+    announce("resident handles on four threads")
+    lang, mid = sh.Langevin(0.02, damping=0.1, kT=0.3), sh.ImplicitMidpoint(0.02)
+
+    def models():
+        out = [sh.workloads.pyrochlore_model(L=12, seed=40 + r, precision=64) for r in range(4)]
+        for s in out:
+            assert s._device().query("cooperative") == 1
+        return out
+
+    def work(s):
+        for _ in range(3):
+            sh.step_(s, lang, nsteps=40)
+            sh.step_(s, mid, nsteps=2)
+
+    one = models()
+    for s in one:
+        work(s)
+    many = models()
+    threads = [threading.Thread(target=work, args=(s,)) for s in many]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for a, b in zip(one, many):
+        assert b._device().query("resident_calls") == 6 and b._device().query("cooperative") == 1
+        np.testing.assert_array_equal(b.dipoles_flat(), a.dipoles_flat())
+
+
 def next_calls():
     """What a program may do after a Langevin call: reads of the state, and
     everything that changes it."""
